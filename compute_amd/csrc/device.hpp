@@ -134,22 +134,22 @@ BDEV uint64_t lb_load(const uint64_t *p)
     return __hip_atomic_load(const_cast<uint64_t *>(p), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 
-// Epoch of a look-back launch.  Before a sequence of L look-back launches
-// the host enqueues k_epoch_advance(L) (one thread: ctrl->epoch += L); launch
-// j of the sequence passes back = L - j and tags its words with
-// ((epoch - back) mod (2^30 - 1)) + 1, so every launch on the queue gets a
-// distinct non-zero epoch, graph replays included.  No per-block atomic is
-// involved: device-scope atomics on one address serialise across XCDs.
+// Epoch of a look-back launch, from its argument (Epochs::arg).  An eager
+// launch is handed the epoch itself.  In a graph the arguments are fixed, so
+// the capture records k_epoch_advance(L) (one thread: ctrl->epoch += L) before
+// L launches, launch j of them takes L - j as its argument, and every replay
+// gets distinct non-zero epochs.  No per-block atomic is involved: device-
+// scope atomics on one address serialise across XCDs.
 //
-// The epoch is a plain load at kernel entry.  ctrl->epoch is written
-// only by k_epoch_advance, an earlier kernel on the same stream, so it is
-// constant for this launch and visible to an ordinary load; with a uniform
-// address that load can be served by the scalar cache, off the vector
-// memory path the tile's data uses.
-BDEV uint32_t launch_epoch_plain(const Ctrl *ctrl, uint32_t back)
+// ctrl->epoch is read with a plain load at kernel entry.  It is written only
+// by k_epoch_advance, an earlier kernel on the same stream, so it is constant
+// for this launch and visible to an ordinary load; with a uniform address
+// that load can be served by the scalar cache, off the vector memory path the
+// tile's data uses.
+BDEV uint32_t launch_epoch(const Ctrl *ctrl, uint32_t arg)
 {
-    const uint32_t e = ctrl->epoch;
-    return ((e - back) % kEpochMask) + 1u;
+    if (arg & kEpochHostArg) return arg & ~kEpochHostArg;
+    return ((ctrl->epoch - arg) % (kEpochSplit - 1u)) + 1u;
 }
 
 // Tiles are numbered by blockIdx.x.  Workgroups are dispatched in id order,

@@ -384,7 +384,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(WPE))) 
 {
     __shared__ QSweepLds<THREADS, IPT, KB, VB, SPLIT> lds;
     const uint32_t tile = xcd_tile(blockIdx.x, xrun);
-    const uint32_t epoch = launch_epoch_plain(ctrl, back);
+    const uint32_t epoch = launch_epoch(ctrl, back);
     if ((uint64_t)(tile + 1) * (THREADS * IPT) <= n)
         qsweep_body<THREADS, IPT, KB, VB, SPLIT, LB, XF, true, CBG>(lds, kin, kout, vin, vout, n, tile, shift,
                                                            ctrl->offsets[pass], xf, ctrl, status, epoch);

@@ -226,7 +226,7 @@ BDEV void onesweep_body(OnesweepLds<KB, VB, IPT> &L, const KB *__restrict__ kin,
     // per digit (thread tid == digit): wave prefixes and the tile count
     const uint32_t c0 = L.cnt[0][tid], c1 = L.cnt[1][tid], c2 = L.cnt[2][tid], c3 = L.cnt[3][tid];
     const uint32_t total = c0 + c1 + c2 + c3;
-    const uint32_t epoch = launch_epoch_plain(ctrl, back);
+    const uint32_t epoch = launch_epoch(ctrl, back);
     if (tile == 0) lb_store(&status[tid], lb_word(epoch, LB_P, total));
     else lb_store(&status[(size_t)tile * 256 + tid], lb_word(epoch, LB_A, total));
     uint32_t inc = wave_inclusive_scan(total, 0u, [](uint32_t a, uint32_t b) { return a + b; });

@@ -348,14 +348,15 @@ static int radix_sort_xf(bcmi_queue q, void *keys_, void *vals_, uint32_t n, XF 
     BCMI_LAUNCH(q, "radix_digit_offsets",
                 hipLaunchKernelGGL(k_digit_offsets, dim3(P), dim3(1024), 0, q->stream, partial, hblocks,
                                    (uint32_t)P, q->ctrl));
-    BCMI_TRY(begin_lookback(q, P));
+    Epochs ep;
+    BCMI_TRY(begin_lookback(q, P, &ep));
     KB *ks = keys, *kd = ktmp;
     V *vs = vals, *vd = vtmp;
     for (int p = 0; p < P; ++p) {
         BCMI_LAUNCH(q, "radix_onesweep",
                     hipLaunchKernelGGL((k_qsweep<TH, IPT, KB, VB, SPLIT, LB, WPE, XF, CBG>), dim3(tiles), dim3(TH), 0, q->stream, ks, kd,
                                        vs, vd, n, (uint32_t)(8 * p), (uint32_t)p, xf, q->ctrl, status,
-                                       (uint32_t)(P - p), (uint32_t)xrun));
+                                       ep.arg((uint32_t)p), (uint32_t)xrun));
         std::swap(ks, kd);
         std::swap(vs, vd);
     }

@@ -124,18 +124,27 @@ __global__ void k_epoch_advance(Ctrl *ctrl, uint32_t count)
     }
 }
 
-int begin_lookback(bcmi_queue q, int launches)
+int begin_lookback(bcmi_queue q, int launches, Epochs *epochs)
 {
-    // Tags carry a 30-bit epoch; clear the status words well before an
-    // epoch value can repeat.
-    if (q->capturing) {
-        q->capture_lookback_launches += (uint64_t)launches;
-    } else {
+    // the stream itself is asked: it may be captured through
+    // bcmi_queue_native as well as by bcmi_graph_begin
+    hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+    BCMI_HIP(hipStreamIsCapturing(q->stream, &cap));
+    if (cap == hipStreamCaptureStatusNone) {
         q->lookback_launches += (uint64_t)launches;
-        if (q->lookback_launches > (1ull << 29)) BCMI_TRY(zero_status(q));
+        if (q->lookback_launches > kEpochClear) {
+            BCMI_TRY(zero_status(q));
+            q->lookback_launches = (uint64_t)launches;
+        }
+        *epochs = Epochs{q->host_epoch, true};
+        q->host_epoch = (q->host_epoch + (uint32_t)launches) % kEpochHostCount;
+        return 0;
     }
+    if (q->capturing) q->capture_lookback_launches += (uint64_t)launches;
+    else q->lookback_launches += (uint64_t)launches;
     hipLaunchKernelGGL(k_epoch_advance, dim3(1), dim3(64), 0, q->stream, q->ctrl, (uint32_t)launches);
     BCMI_HIP(hipGetLastError());
+    *epochs = Epochs{(uint32_t)launches, false};
     return 0;
 }
 
@@ -502,7 +511,7 @@ int bcmi_graph_launch(bcmi_graph g, bcmi_queue q)
                "needed more); reserve enough with bcmi_queue_reserve before capturing, then capture again");
     BCMI_HIP(hipGraphLaunch(g->exec, q->stream));
     q->lookback_launches += g->lookback_launches;
-    if (q->lookback_launches > (1ull << 29)) BCMI_TRY(zero_status(q));
+    if (q->lookback_launches > kEpochClear) BCMI_TRY(zero_status(q));
     return 0;
 }
 

@@ -12,9 +12,9 @@
 //     graph records the generation it was captured under and refuses to
 //     replay once it changed, since its kernels hold the freed addresses;
 //   * a look-back status array (decoupled look-back scans and onesweep
-//     digit offsets).  Status words are tagged with an epoch that the last
-//     block of every look-back kernel advances on the device, so the array
-//     is never cleared between calls and graph replays stay correct;
+//     digit offsets).  Status words are tagged with the launch's epoch
+//     (numbered by the host, or on the device for graph replays), so the
+//     array is never cleared between calls and replays stay correct;
 //   * a small device control block: the look-back epoch, a fault flag and
 //     the radix digit offsets of the current sort.
 #pragma once
@@ -33,14 +33,34 @@ namespace bcmi {
 
 // Device control block, zero-initialised at queue creation.
 struct Ctrl {
-    uint32_t epoch;          // look-back epoch counter (advanced by k_epoch_advance)
+    uint32_t epoch;          // look-back epoch counter of captured launches (advanced by k_epoch_advance)
     uint32_t fault;          // set by a kernel whose look-back wait expired or whose output index was out of range
     uint32_t spin_limit;     // polls before a look-back wait gives up; 0: kSpinLimit (tests lower it)
     uint32_t never_set;      // written by no kernel and no host code: the fault probe's wait target
     uint32_t offsets[8][256];// exclusive digit offsets per radix pass
 };
 
-constexpr uint32_t kEpochMask = (1u << 30) - 1u;
+// Look-back epochs (30 bits, 0 = never published).  [1, kEpochSplit) are the
+// device's: ctrl->epoch, advanced by a kernel, for launches recorded in a
+// graph, whose arguments stay as they were at every replay.  [kEpochSplit,
+// 2^30) are the host's: an eager launch carries its epoch as an argument, so
+// nothing has to run before it (the one-thread advance kernel took 1.5-4.8 us
+// of GPU time in front of every look-back call).
+constexpr uint32_t kEpochSplit = 3u << 28;
+constexpr uint32_t kEpochHostCount = (1u << 30) - kEpochSplit;
+constexpr uint32_t kEpochHostArg = 1u << 31;  // tag of a launch argument that is the epoch itself
+// status words are cleared after this many launches, long before either range repeats
+constexpr uint64_t kEpochClear = 1ull << 27;
+
+// The epochs of a sequence of look-back launches: launch j passes arg(j).
+struct Epochs {
+    uint32_t first;  // host: epoch index of launch 0; device: the number of launches
+    bool host;
+    uint32_t arg(uint32_t j) const
+    {
+        return host ? (kEpochHostArg | (kEpochSplit + (first + j) % kEpochHostCount)) : first - j;
+    }
+};
 
 struct ProfRec {
     const char *name;
@@ -61,7 +81,8 @@ struct bcmi_queue_s {
     // look-back status words (uint64)
     uint64_t *status = nullptr;
     size_t status_words = 0;
-    uint64_t lookback_launches = 0;
+    uint64_t lookback_launches = 0;  // since the status words were last cleared
+    uint32_t host_epoch = 0;         // index of the next host-numbered look-back launch
     // bumped whenever scratch or status is reallocated
     uint64_t arena_gen = 0;
     // control block
@@ -117,9 +138,10 @@ int use_queue(bcmi_queue q);
 int scratch(bcmi_queue q, size_t bytes, void **ptr);
 // Look-back status array of at least `words` uint64.
 int status_array(bcmi_queue q, size_t words, uint64_t **ptr);
-// Reserve epochs for the next `launches` look-back launches on the queue:
-// enqueues the epoch advance and does the wrap bookkeeping.
-int begin_lookback(bcmi_queue q, int launches);
+// Reserve epochs for the next `launches` look-back launches on the queue and
+// do the wrap bookkeeping.  While the stream is being captured it enqueues
+// the device's epoch advance; otherwise it enqueues nothing.
+int begin_lookback(bcmi_queue q, int launches, Epochs *epochs);
 
 // Profiling brackets around a kernel launch on q->stream.
 void prof_begin(bcmi_queue q, const char *name, ProfRec *rec);

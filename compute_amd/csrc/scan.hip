@@ -374,7 +374,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE))) 
         __shared__ uint32_t rows[NW * RowShape<Q, BG>::WORDS];
         blk = rows;
     }
-    const uint32_t epoch = launch_epoch_plain(ctrl, back);
+    const uint32_t epoch = launch_epoch(ctrl, back);
     if ((size_t)(blockIdx.x + 1) * TILE <= n)
         scan_body<T, P, VEC, Q, NW, true, BG>(lds, blk, src, out, n, ctrl, status, init, exclusive, epoch);
     else
@@ -389,15 +389,16 @@ static int launch_scan(bcmi_queue q, const Src &src, T *out, size_t n, uint64_t 
     size_t tiles = (n + TILE - 1) / TILE;
     BCMI_CHECK(tiles < (1ull << 31), BCMI_INVALID_BUFFER_SIZE, "scan: n=%zu too large", n);
     bool vec = (((uintptr_t)src.ptr | (uintptr_t)out) & 15) == 0;
-    BCMI_TRY(begin_lookback(q, 1));
+    Epochs ep;
+    BCMI_TRY(begin_lookback(q, 1, &ep));
     if (vec) {
         BCMI_LAUNCH(q, "scan",
                     hipLaunchKernelGGL((k_scan<T, P, true, Q, Src, NW, BG, WPE>), dim3((unsigned)tiles), dim3(NW * 64), 0,
-                                       q->stream, src, out, n, q->ctrl, status, ini, exclusive, 1u));
+                                       q->stream, src, out, n, q->ctrl, status, ini, exclusive, ep.arg(0)));
     } else {
         BCMI_LAUNCH(q, "scan",
                     hipLaunchKernelGGL((k_scan<T, P, false, Q, Src, NW, BG, WPE>), dim3((unsigned)tiles), dim3(NW * 64), 0,
-                                       q->stream, src, out, n, q->ctrl, status, ini, exclusive, 1u));
+                                       q->stream, src, out, n, q->ctrl, status, ini, exclusive, ep.arg(0)));
     }
     return 0;
 }

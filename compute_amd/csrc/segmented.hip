@@ -376,7 +376,7 @@ __global__ __launch_bounds__(kSortThreads) void k_qsweep_seg(const KB *__restric
     __shared__ QSweepLds<kSortThreads, IPT, KB, VB, 1> lds;
     const SegTile t = tiles[blockIdx.x];
     if (t.route != want) return;  // the segment takes the other route
-    const uint32_t epoch = launch_epoch_plain(ctrl, back);
+    const uint32_t epoch = launch_epoch(ctrl, back);
     const size_t b = t.base;
     const uint32_t *goff = seg_off + ((size_t)t.seg * passes + pass) * 256;
     uint64_t *st = status + (size_t)(blockIdx.x - t.tile) * 256;
@@ -602,7 +602,8 @@ static int run_plan_large(bcmi_queue q, bcmi_segplan pl, KB *keys, typename ValT
         }
         uint64_t *status;
         BCMI_TRY(status_array(q, (size_t)pl->ntiles * 256, &status));
-        BCMI_TRY(begin_lookback(q, P + 1));
+        Epochs ep;
+        BCMI_TRY(begin_lookback(q, P + 1, &ep));
         // MSD route: top-digit partition into the temporaries ...
         // (param "qrank" = 1: the quarter-wave pass body)
 #define BCMI_SEG_PASS(NAME, KS, KD, VS, VD, SHIFT, PASS, BACK, WANT)                                            \
@@ -621,7 +622,7 @@ static int run_plan_large(bcmi_queue q, bcmi_segplan pl, KB *keys, typename ValT
                                                BACK, WANT));                                                    \
         } while (0)
         BCMI_SEG_PASS("segsort_onesweep_msd", keys, (KB *)pl->ktmp, vals, (V *)pl->vtmp, (uint32_t)(8 * (P - 1)),
-                      (uint32_t)(P - 1), (uint32_t)(P + 1), (uint32_t)kRouteMsd);
+                      (uint32_t)(P - 1), ep.arg(0), (uint32_t)kRouteMsd);
         // ... then every group sorted in LDS from the temporaries back into place
 #define BCMI_GROUPS(CLS, IPTV)                                                                                  \
     if constexpr ((int)(sizeof(KB) + VB) * kSegSmallThreads * IPTV <= kSegSmallLds) {                           \
@@ -641,7 +642,7 @@ static int run_plan_large(bcmi_queue q, bcmi_segplan pl, KB *keys, typename ValT
         KB *ks = keys, *kd = (KB *)pl->ktmp;
         V *vs = vals, *vd = (V *)pl->vtmp;
         for (int p = 0; p < P; ++p) {
-            BCMI_SEG_PASS("segsort_onesweep", ks, kd, vs, vd, (uint32_t)(8 * p), (uint32_t)p, (uint32_t)(P - p),
+            BCMI_SEG_PASS("segsort_onesweep", ks, kd, vs, vd, (uint32_t)(8 * p), (uint32_t)p, ep.arg((uint32_t)p + 1),
                           (uint32_t)kRouteLsd);
             std::swap(ks, kd);
             std::swap(vs, vd);

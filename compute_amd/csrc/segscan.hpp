@@ -501,7 +501,7 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 8
 {
     constexpr size_t TILE = (size_t)NW * Q * 64 * (16 / sizeof(VT));
     const bool full = (size_t)(blockIdx.x + 1) * TILE <= n;
-    const uint32_t epoch = launch_epoch_plain(ctrl, back);
+    const uint32_t epoch = launch_epoch(ctrl, back);
     if constexpr (sizeof(KT) == 4 && sizeof(VT) == 4 && Q <= 8) {
         __shared__ SegLdsBlk<P, Q, NW> lds;
         if (full)
@@ -529,17 +529,18 @@ static int launch_seg(bcmi_queue q, const void *keys, const void *vals, void *ou
     constexpr size_t TILE = (size_t)NW * Q * 64 * (16 / sizeof(VT));
     size_t tiles = (n + TILE - 1) / TILE;
     const bool vec = (((uintptr_t)keys | (uintptr_t)vals | (MODE == SEG_RBK ? 0 : (uintptr_t)out)) & 15) == 0;
-    BCMI_TRY(begin_lookback(q, 1));
+    Epochs ep;
+    BCMI_TRY(begin_lookback(q, 1, &ep));
     if (vec)
         BCMI_LAUNCH(q, MODE == SEG_RBK ? "reduce_by_key" : "segmented_scan",
                     hipLaunchKernelGGL((k_segscan<KT, VT, P, MODE, Q, true, NW>), dim3((unsigned)tiles),
                                        dim3(NW * 64), 0, q->stream, (const KT *)keys, (const VT *)vals, (VT *)out,
-                                       (KT *)keys_out, n, q->ctrl, status, ini, count_out, 1u));
+                                       (KT *)keys_out, n, q->ctrl, status, ini, count_out, ep.arg(0)));
     else
         BCMI_LAUNCH(q, MODE == SEG_RBK ? "reduce_by_key" : "segmented_scan",
                     hipLaunchKernelGGL((k_segscan<KT, VT, P, MODE, Q, false, NW>), dim3((unsigned)tiles),
                                        dim3(NW * 64), 0, q->stream, (const KT *)keys, (const VT *)vals, (VT *)out,
-                                       (KT *)keys_out, n, q->ctrl, status, ini, count_out, 1u));
+                                       (KT *)keys_out, n, q->ctrl, status, ini, count_out, ep.arg(0)));
     return 0;
 }
 

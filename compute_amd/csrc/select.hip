@@ -384,7 +384,7 @@ __global__ __launch_bounds__(kSelThreads) __attribute__((amdgpu_waves_per_eu(BCM
     constexpr size_t TILE = SelShape<T>::TILE;
     __shared__ SelLds<T, MODE> lds;
     const size_t tstart = (size_t)blockIdx.x * TILE;
-    const uint32_t epoch = launch_epoch_plain(ctrl, back);
+    const uint32_t epoch = launch_epoch(ctrl, back);
     if (tstart >= head && tstart + TILE <= head + n)
         select_body<T, MODE, true>(lds, abase, head, n, out_a, out_b, p, ctrl, status, count_out, epoch);
     else
@@ -534,10 +534,11 @@ static int launch_select(bcmi_queue q, const T *in, void *out_a, void *out_b, si
     BCMI_CHECK(tiles < (1ull << 31), BCMI_INVALID_BUFFER_SIZE, "select: n=%zu too large", n);
     uint64_t *status;
     BCMI_TRY(status_array(q, tiles + 1, &status));
-    BCMI_TRY(begin_lookback(q, 1));
+    Epochs ep;
+    BCMI_TRY(begin_lookback(q, 1, &ep));
     BCMI_LAUNCH(q, "select",
                 hipLaunchKernelGGL((k_select<T, MODE>), dim3((unsigned)tiles), dim3(kSelThreads), 0, q->stream,
-                                   abase, head, n, out_a, out_b, p, q->ctrl, status, count_out, 1u));
+                                   abase, head, n, out_a, out_b, p, q->ctrl, status, count_out, ep.arg(0)));
     return 0;
 }
 
