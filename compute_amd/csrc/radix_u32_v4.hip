@@ -1,0 +1,11 @@
+// Instantiation unit of radix_sort.hpp.
+#include "radix_sort.hpp"
+
+namespace bcmi {
+
+BCMI_RADIX_SIGNATURE(radix_keys_u32_v4)
+{
+    return radix_sort_shape<uint32_t, 4>(q, keys, vals, n, kind, desc, work);
+}
+
+}  // namespace bcmi
