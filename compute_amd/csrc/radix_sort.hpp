@@ -270,46 +270,64 @@ static int radix_sort(bcmi_queue q, void *keys, void *vals, uint32_t n, int kind
     });
 }
 
-// Tile shape: threads per workgroup, keys per thread and staging rounds.
-// For 4-byte keys with no or 4-byte values it comes from the tuning cache
-// (key "__bcmi_radix_sort", or "__bcmi_radix_sort_by_key" with values;
-// params "threads", "ipt", "split", "lookback" (predecessor words per
-// look-back round trip) and "waves" (a register bound, waves per SIMD; 0 =
-// none), "count_bg" (1: bank-grouped count words, built for the best
-// shapes), chosen on 2^27 keys; the lookback / waves combinations built are
-// listed below; smaller sorts take
-// smaller tiles to fill the chip (param "fit_size" = 0 keeps the tuned shape
-// at every size).  Other key and value widths take a fixed shape whose
-// staging buffer stays within 32-64 KB (two workgroups per CU).
+// Tile shape: threads per workgroup, keys per thread, staging rounds and
+// predecessor words per look-back round trip, by the number of keys.
+//
+// A pass over a few hundred tiles is bound by one tile's chain of latencies
+// (load, count, scan, rank, look-back, scattered store), so small sorts take
+// tiles of 4096 keys held by many threads with few keys each (the ranking
+// chain is 3 dependent LDS round trips per key of a thread), and tiles grow
+// with n: a longer digit run per tile writes fuller lines, and half the tiles
+// are half the look-backs.  Each line below lies where the two sides met; us
+// a call with the copy of the input, smaller tile first.
+//   uint32            512 x 8 | 512 x 16     2^18: 46.5 47.5   2^19: 56.3 54.6
+//                     512 x 16 | 1024 x 16   2^21: 84.7 85.6   4 M: 107 100
+//                     1024 x 16 | tuned      8 M: 137 141 (512 x 32)   16 M: 212 204
+//   float + u32       512 x 8 | 512 x 16     2^20: 81.7 84.4   2^21: over 104, 98.9
+//                     512 x 16 | tuned       4 M: 132 134   8 M: 204 195
+//   uint64            512 x 8 | 512 x 16     2^18: 91 98   2^20: 144 142
+//                     512 x 16 | 512 x 32    4 M: 223 over 224   8 M: over 328, 305
+//   uint64 + u32      512 x 8 | 512 x 16     2^20: 153 158   1.5 M: 179 171
+//   8-byte values: the last two lines' shapes; at 8 M and more their tiles
+//   are staged in two rounds and grouped by XCD (uint64 + u32 8 M: 480 437).
+// (256 x 16 up to 2^20 and 256 x 32 up to 2^23 before: uint32 73.2 at 2^20,
+// 156 at 8 M; uint64, always 256 x 16, 410 at 8 M and 792 at 16 M.)
+//
+// Above those sizes 4-byte keys with no or 4-byte values take the shape of
+// the tuning cache (key "__bcmi_radix_sort", or "__bcmi_radix_sort_by_key"
+// with values; params "threads", "ipt", "split", "lookback", "waves" (a
+// register bound, waves per SIMD; 0 = none) and "count_bg" (1: bank-grouped
+// count words)), chosen on 2^27 keys; the combinations built are listed
+// below.  Param "fit_size" = 0 keeps the tuned shape at every size.  1- and
+// 2-byte keys and other value widths take a fixed shape.  The allocation-free
+// sort (work != nullptr) reads no tuning cache and keeps to the two smallest
+// shapes.
 template <typename KB, int VB>
 static int radix_sort_shape(bcmi_queue q, void *keys, void *vals, uint32_t n, int kind, int desc,
                             const SortWork *work)
 {
     constexpr int SB = (int)sizeof(KB) > VB ? (int)sizeof(KB) : VB;
-    // the allocation-free sort (work != nullptr) reads no tuning cache
     const char *key = VB ? "__bcmi_radix_sort_by_key" : "__bcmi_radix_sort";
     const unsigned xrun = work ? 0u : tune_get(key, "xcd_run", 0);
     if constexpr (sizeof(KB) == 4 && (VB == 0 || VB == 4)) {
-        unsigned th = work ? 256 : tune_get(key, "threads", 512);
-        unsigned ipt = work ? 32 : tune_get(key, "ipt", 32);
-        unsigned split = work ? 1 : tune_get(key, "split", 1);
-        const unsigned lb = work ? 4 : tune_get(key, "lookback", 4);
-        const unsigned wpe = work ? 0 : tune_get(key, "waves", 0);
-        const unsigned cbg = work ? 0 : tune_get(key, "count_bg", 0);
-        bool tuned_shape = true;
         if (work || tune_get(key, "fit_size", 1) != 0) {
-            if (n <= (1u << 20)) {
-                th = 256;
-                ipt = 16;
-                split = 1;
-                tuned_shape = false;
-            } else if (n <= (1u << 23)) {
-                th = 256;
-                ipt = 32;
-                split = 1;
-                tuned_shape = false;
+            if (n <= (VB ? 1u << 20 : 1u << 18))
+                return radix_sort<KB, VB, 512, 8, 1, 8>(q, keys, vals, n, kind, desc, work, 0);
+            if constexpr (VB == 0) {
+                if (work || n <= 2500000)
+                    return radix_sort<KB, VB, 512, 16, 1, 8>(q, keys, vals, n, kind, desc, work, 0);
+                if (n <= 12000000) return radix_sort<KB, VB, 1024, 16, 1, 8>(q, keys, vals, n, kind, desc, work, 0);
+            } else {
+                if (work || n <= 5000000)
+                    return radix_sort<KB, VB, 512, 16, 2, 4, 1, 1>(q, keys, vals, n, kind, desc, work, 0);
             }
         }
+        const unsigned th = tune_get(key, "threads", 512);
+        const unsigned ipt = tune_get(key, "ipt", 32);
+        const unsigned split = tune_get(key, "split", 1);
+        const unsigned lb = tune_get(key, "lookback", 4);
+        const unsigned wpe = tune_get(key, "waves", 0);
+        const unsigned cbg = tune_get(key, "count_bg", 0);
         // register bounds (param "waves": waves per SIMD) that raise the
         // workgroups per CU to what the LDS allows without spills, and
         // look-back windows other than 4 words per round trip, for the
@@ -324,22 +342,20 @@ static int radix_sort_shape(bcmi_queue q, void *keys, void *vals, uint32_t n, in
         if constexpr (sizeof(QSweepLds<T, I, KB, VB, S>) <= (size_t)kLdsBytesPerCU)                         \
             if (th == T && ipt == I && split == S && lb == W && wpe == E && cbg == 1)                      \
                 return radix_sort<KB, VB, T, I, S, W, E, 1>(q, keys, vals, n, kind, desc, work, xrun)
-        if (tuned_shape) {
-            BCMI_SHAPE_CB(512, 64, 2, 2, 4);
-            BCMI_SHAPE_CB(256, 64, 2, 2, 4);
-            BCMI_SHAPE_CB(512, 32, 2, 2, 0);
-            BCMI_SHAPE_CB(512, 32, 2, 2, 7);
-            BCMI_SHAPE_LB(256, 64, 2, 2, 0);
-            BCMI_SHAPE_LB(512, 32, 2, 2, 0);
-            BCMI_SHAPE_LB(256, 64, 2, 2, 4);
-            BCMI_SHAPE_LB(512, 24, 2, 2, 8);
-            BCMI_SHAPE_LB(512, 32, 2, 2, 7);
-            BCMI_SHAPE_LB(512, 16, 1, 4, 8);
-            BCMI_SHAPE_LB(512, 64, 2, 2, 4);
-            BCMI_SHAPE_LB(512, 64, 4, 2, 4);
-            BCMI_SHAPE_LB(1024, 32, 2, 2, 0);
-            BCMI_SHAPE_LB(1024, 32, 4, 2, 0);
-        }
+        BCMI_SHAPE_CB(512, 64, 2, 2, 4);
+        BCMI_SHAPE_CB(256, 64, 2, 2, 4);
+        BCMI_SHAPE_CB(512, 32, 2, 2, 0);
+        BCMI_SHAPE_CB(512, 32, 2, 2, 7);
+        BCMI_SHAPE_LB(256, 64, 2, 2, 0);
+        BCMI_SHAPE_LB(512, 32, 2, 2, 0);
+        BCMI_SHAPE_LB(256, 64, 2, 2, 4);
+        BCMI_SHAPE_LB(512, 24, 2, 2, 8);
+        BCMI_SHAPE_LB(512, 32, 2, 2, 7);
+        BCMI_SHAPE_LB(512, 16, 1, 4, 8);
+        BCMI_SHAPE_LB(512, 64, 2, 2, 4);
+        BCMI_SHAPE_LB(512, 64, 4, 2, 4);
+        BCMI_SHAPE_LB(1024, 32, 2, 2, 0);
+        BCMI_SHAPE_LB(1024, 32, 4, 2, 0);
 #undef BCMI_SHAPE_LB
 #undef BCMI_SHAPE_CB
 #define BCMI_SHAPE(T, I, S) \
@@ -357,6 +373,13 @@ static int radix_sort_shape(bcmi_queue q, void *keys, void *vals, uint32_t n, in
         BCMI_SHAPE(512, 24, 3);
 #undef BCMI_SHAPE
         // any other value falls through to the generic shape below
+    }
+    if constexpr ((sizeof(KB) == 8 && (VB == 0 || VB == 4 || VB == 8)) || (sizeof(KB) == 4 && VB == 8)) {
+        if (work || n <= (VB ? 1u << 20 : 1u << 19))
+            return radix_sort<KB, VB, 512, 8, 1, 8>(q, keys, vals, n, kind, desc, work, 0);
+        if (n <= 6000000) return radix_sort<KB, VB, 512, 16, 1, 8>(q, keys, vals, n, kind, desc, work, 0);
+        if constexpr (VB == 0) return radix_sort<KB, VB, 512, 32, 2, 2>(q, keys, vals, n, kind, desc, work, xrun);
+        else return radix_sort<KB, VB, 512, 16, 2, 4>(q, keys, vals, n, kind, desc, work, xrun);
     }
     if constexpr (SB >= 8) return radix_sort<KB, VB, 256, 16>(q, keys, vals, n, kind, desc, work, xrun);
     else return radix_sort<KB, VB, 256, 32>(q, keys, vals, n, kind, desc, work, xrun);
