@@ -25,9 +25,10 @@ namespace bcmi {
 
 // One block of 1024 threads per pass: thread (slice, d) sums digit d over a
 // quarter of the partial histograms, the slices are combined in LDS and the
-// 256 totals scanned into exclusive digit offsets.
+// 256 totals scanned into exclusive digit offsets.  A pass whose digit is the
+// same in all n keys is marked in ctrl->single.
 __global__ __launch_bounds__(1024) void k_digit_offsets(const uint32_t *__restrict__ partial, uint32_t nparts,
-                                                        uint32_t passes, Ctrl *ctrl)
+                                                        uint32_t passes, uint32_t n, Ctrl *ctrl)
 {
     __shared__ uint32_t s_part[4][256];
     __shared__ uint32_t s_wsum[4];
@@ -41,7 +42,8 @@ __global__ __launch_bounds__(1024) void k_digit_offsets(const uint32_t *__restri
     c = s_part[0][d] + s_part[1][d] + s_part[2][d] + s_part[3][d];
     uint32_t inc = wave_inclusive_scan(c, 0u, [](uint32_t a, uint32_t b) { return a + b; });
     if (slice == 0 && lane == 63) s_wsum[w] = inc;
-    block_barrier();
+    const int single = block_barrier_or(c == n);
+    if (threadIdx.x == 0) ctrl->single[p] = single ? 1u : 0u;
     if (slice == 0) {
         uint32_t pre = 0;
         for (uint32_t i = 0; i < w; ++i) pre += s_wsum[i];

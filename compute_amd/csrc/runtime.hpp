@@ -38,6 +38,7 @@ struct Ctrl {
     uint32_t spin_limit;     // polls before a look-back wait gives up; 0: kSpinLimit (tests lower it)
     uint32_t never_set;      // written by no kernel and no host code: the fault probe's wait target
     uint32_t offsets[8][256];// exclusive digit offsets per radix pass
+    uint32_t single[8];      // per radix pass: every key has the same digit
 };
 
 // Look-back epochs (30 bits, 0 = never published).  [1, kEpochSplit) are the

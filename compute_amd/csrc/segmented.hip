@@ -364,9 +364,9 @@ void k_onesweep_seg(const KB *__restrict__ kin, KB *__restrict__ kout,
 // staged while its look-back completes.  Tile, look-back chain and offsets
 // are the segment's, as above.
 template <typename KB, int VB, int IPT, typename XF>
-__global__ __launch_bounds__(kSortThreads) void k_qsweep_seg(const KB *__restrict__ kin, KB *__restrict__ kout,
-                                                             const typename ValT<VB>::type *__restrict__ vin,
-                                                             typename ValT<VB>::type *__restrict__ vout,
+__global__ __launch_bounds__(kSortThreads) void k_qsweep_seg(KB *kin, KB *kout,
+                                                             typename ValT<VB>::type *vin,
+                                                             typename ValT<VB>::type *vout,
                                                              const SegTile *__restrict__ tiles, uint32_t shift,
                                                              uint32_t pass, uint32_t passes,
                                                              const uint32_t *__restrict__ seg_off, XF xf,
@@ -383,11 +383,11 @@ __global__ __launch_bounds__(kSortThreads) void k_qsweep_seg(const KB *__restric
     if ((uint64_t)(t.tile + 1) * (kSortThreads * IPT) <= t.len)
         qsweep_body<kSortThreads, IPT, KB, VB, 1, 2, XF, true, 1>(lds, kin + b, kout + b, VB ? vin + b : vin,
                                                                 VB ? vout + b : vout, t.len, t.tile, shift, goff, xf,
-                                                                ctrl, st, epoch);
+                                                                ctrl, st, epoch, PlainPass());
     else
         qsweep_body<kSortThreads, IPT, KB, VB, 1, 2, XF, false, 1>(lds, kin + b, kout + b, VB ? vin + b : vin,
                                                                  VB ? vout + b : vout, t.len, t.tile, shift, goff,
-                                                                 xf, ctrl, st, epoch);
+                                                                 xf, ctrl, st, epoch, PlainPass());
 }
 
 // One block (256 threads, thread = digit) per large segment.  The top-digit
