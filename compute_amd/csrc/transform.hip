@@ -46,81 +46,59 @@ struct BinOp {
     }
 };
 
-// Vector body over whole 16-byte chunks; the caller guarantees a, b and out
-// are 16-byte aligned.
-template <typename T, typename F>
-__global__ __launch_bounds__(kTfThreads) void k_transform_vec(const vec16<T> *__restrict__ a,
-                                                              const vec16<T> *__restrict__ b,
-                                                              vec16<T> *__restrict__ out, size_t nchunks, F f)
+// U 16-byte chunks of every operand per thread, and the elements after the
+// last whole chunk in the thread that would have had the next one: one launch
+// for any n.  vec16 is aligned as its elements are: a wave's chunks are one
+// contiguous 1 KB either way, and off the 16-byte grid it only touches one
+// line more.  Bound by HBM from a few MB on; saxpy us a call: 4 M floats 9.1 ->
+// 7.3, 10 M 26.5 -> 19 (a second launch served the tail), 1001 floats off the
+// grid 9.6 -> 4.1 (the element-wise path that served such operands).
+template <typename T, typename F, int U>
+__global__ __launch_bounds__(kTfThreads) void k_transform(const T *__restrict__ a, const T *__restrict__ b,
+                                                          T *__restrict__ out, size_t n, F f)
 {
-    size_t base = (size_t)blockIdx.x * (kTfThreads * kTfUnroll) + threadIdx.x;
-    vec16<T> va[kTfUnroll], vb[kTfUnroll];
+    constexpr int N = vec16<T>::N;
+    const size_t nchunks = n / N;
+    const size_t base = (size_t)blockIdx.x * (kTfThreads * U) + threadIdx.x;
+    vec16<T> va[U], vb[U];
 #pragma unroll
-    for (int j = 0; j < kTfUnroll; ++j) {
-        size_t c = base + (size_t)j * kTfThreads;
+    for (int j = 0; j < U; ++j) {
+        const size_t c = base + (size_t)j * kTfThreads;
         if (c < nchunks) {
-            va[j] = a[c];
-            vb[j] = b[c];
+            va[j] = *(const vec16<T> *)(a + c * N);
+            vb[j] = *(const vec16<T> *)(b + c * N);
         }
     }
 #pragma unroll
-    for (int j = 0; j < kTfUnroll; ++j) {
-        size_t c = base + (size_t)j * kTfThreads;
+    for (int j = 0; j < U; ++j) {
+        const size_t c = base + (size_t)j * kTfThreads;
         if (c < nchunks) {
             vec16<T> r;
 #pragma unroll
-            for (int k = 0; k < vec16<T>::N; ++k) r.v[k] = f(va[j].v[k], vb[j].v[k]);
-            out[c] = r;
+            for (int k = 0; k < N; ++k) r.v[k] = f(va[j].v[k], vb[j].v[k]);
+            *(vec16<T> *)(out + c * N) = r;
+        } else if (c == nchunks) {
+            for (size_t i = c * N; i < n; ++i) out[i] = f(a[i], b[i]);
         }
     }
-}
-
-// Scalar path for heads/tails and for operands that are not mutually aligned.
-template <typename T, typename F>
-__global__ __launch_bounds__(kTfThreads) void k_transform_scalar(const T *__restrict__ a, const T *__restrict__ b,
-                                                                 T *__restrict__ out, size_t n, F f)
-{
-    size_t i = (size_t)blockIdx.x * kTfThreads + threadIdx.x;
-    size_t stride = (size_t)gridDim.x * kTfThreads;
-    for (; i < n; i += stride) out[i] = f(a[i], b[i]);
 }
 
 template <typename T, typename F>
 static int run_transform(bcmi_queue q, const T *a, const T *b, T *out, size_t n, F f, const char *name)
 {
     if (n == 0) return 0;
-    const uintptr_t mask = 15;
-    size_t head = 0;
-    uintptr_t oa = (uintptr_t)out & mask;
-    bool aligned = (((uintptr_t)a & mask) == oa) && (((uintptr_t)b & mask) == oa) && (oa % sizeof(T) == 0);
-    if (aligned && oa != 0) head = (16 - oa) / sizeof(T);
-    if (head > n) head = n;
-    size_t body = aligned ? (n - head) / vec16<T>::N : 0;
-    size_t done = head + body * vec16<T>::N;
-    int maxb = q->cu_count * 8;
-    if (!aligned) {
-        size_t blocks = (n + kTfThreads - 1) / kTfThreads;
-        if (blocks > (size_t)maxb) blocks = maxb;
-        BCMI_LAUNCH(q, name, hipLaunchKernelGGL((k_transform_scalar<T, F>), dim3((unsigned)blocks), dim3(kTfThreads), 0,
-                                                q->stream, a, b, out, n, f));
-        return 0;
-    }
-    if (head) {
-        BCMI_LAUNCH(q, name, hipLaunchKernelGGL((k_transform_scalar<T, F>), dim3(1), dim3(kTfThreads), 0, q->stream, a,
-                                                b, out, head, f));
-    }
-    if (body) {
-        size_t per = (size_t)kTfThreads * kTfUnroll;
-        size_t blocks = (body + per - 1) / per;
+    const size_t chunks = (n + vec16<T>::N - 1) / vec16<T>::N;  // the last one may be the tail
+    // one chunk per thread until that gives every CU several workgroups
+    const bool small = chunks <= (size_t)q->cu_count * kTfThreads * 8;
+    const size_t per = (size_t)kTfThreads * (small ? 1 : kTfUnroll);
+    const dim3 grid((unsigned)((chunks + per - 1) / per));
+    if (small)
         BCMI_LAUNCH(q, name,
-                    hipLaunchKernelGGL((k_transform_vec<T, F>), dim3((unsigned)blocks), dim3(kTfThreads), 0, q->stream,
-                                       (const vec16<T> *)(a + head), (const vec16<T> *)(b + head),
-                                       (vec16<T> *)(out + head), body, f));
-    }
-    if (done < n) {
-        BCMI_LAUNCH(q, name, hipLaunchKernelGGL((k_transform_scalar<T, F>), dim3(1), dim3(kTfThreads), 0, q->stream,
-                                                a + done, b + done, out + done, n - done, f));
-    }
+                    hipLaunchKernelGGL((k_transform<T, F, 1>), grid, dim3(kTfThreads), 0, q->stream, a, b, out, n, f));
+    else
+        BCMI_LAUNCH(q, name,
+                    hipLaunchKernelGGL((k_transform<T, F, kTfUnroll>), grid, dim3(kTfThreads), 0, q->stream, a, b, out,
+                                       n, f));
     return 0;
 }
 
