@@ -8,7 +8,7 @@
 // (accumulate.hpp:62-69).
 //
 // Here: one streaming pass of a few blocks per CU (as reduce.hip) evaluates
-// the element map while folding, then one block folds the block partials
+// the element map while folding, and its last block folds the block partials
 // in a fixed order.  No temporary.  Compensated float sums keep the exact
 // rounding error of a final product or square (fma), so a float inner
 // product is accurate to about the FP64 result.  Counting sequences are
@@ -59,24 +59,20 @@ BDEV T count_at(int64_t start, size_t i)
     else return (T)((uint64_t)start + (uint64_t)i);
 }
 
-// Two arrays (or one), both at the same offset inside a 16-byte chunk:
-// block 0 takes the head and tail elements, all blocks stream the chunks,
-// two in flight per thread.
+// Two arrays (or one): block 0 takes the elements after the last whole chunk,
+// all blocks stream the chunks, two in flight per thread.
 template <typename T, typename P, int FN, int OPB>
-BDEV typename P::State fold_arrays(const T *a, const T *b, size_t n, size_t head, size_t nchunks, T c)
+BDEV typename P::State fold_arrays(const T *a, const T *b, size_t n, T c)
 {
     using S = typename P::State;
     constexpr int V = chunk16<T>::N;
     S acc = P::id();
-    const size_t tail0 = head + nchunks * V;
-    if (blockIdx.x == 0) {
-        for (size_t i = threadIdx.x; i < head; i += kRedThreads)
+    const size_t nchunks = n / V;
+    if (blockIdx.x == 0)
+        for (size_t i = nchunks * V + threadIdx.x; i < n; i += kRedThreads)
             acc = map_fold<T, P, FN, OPB>(acc, a[i], OPB != kMapUnary ? b[i] : T(0), c);
-        for (size_t i = tail0 + threadIdx.x; i < n; i += kRedThreads)
-            acc = map_fold<T, P, FN, OPB>(acc, a[i], OPB != kMapUnary ? b[i] : T(0), c);
-    }
-    const chunk16<T> *ca = (const chunk16<T> *)(a + head);
-    const chunk16<T> *cb = (const chunk16<T> *)(OPB != kMapUnary ? b + head : a + head);
+    const chunk16<T> *ca = (const chunk16<T> *)a;
+    const chunk16<T> *cb = (const chunk16<T> *)(OPB != kMapUnary ? b : a);
     const size_t stride = (size_t)gridDim.x * kRedThreads;
     size_t i = (size_t)blockIdx.x * kRedThreads + threadIdx.x;
     for (; i + stride < nchunks; i += 2 * stride) {
@@ -117,30 +113,29 @@ BDEV typename P::State fold_general(const T *a, int64_t a0, const T *b, int64_t 
 }
 
 template <typename T, typename P, bool VEC, int OPB, int FN>
-BDEV typename P::State fold_any(const T *a, int64_t a0, const T *b, int64_t b0, size_t n, size_t head,
-                                size_t nchunks, T c)
+BDEV typename P::State fold_any(const T *a, int64_t a0, const T *b, int64_t b0, size_t n, T c)
 {
-    if constexpr (VEC) return fold_arrays<T, P, FN, OPB>(a, b, n, head, nchunks, c);
+    if constexpr (VEC) return fold_arrays<T, P, FN, OPB>(a, b, n, c);
     else return fold_general<T, P, FN, OPB>(a, a0, b, b0, n, c);
 }
 
-// VEC: both inputs are arrays sharing their offset inside a 16-byte chunk.
+// VEC: the inputs are arrays of 4- or 8-byte elements.
 template <typename T, typename P, bool VEC, int OPB>
 __global__ __launch_bounds__(kRedThreads) void k_mapreduce(const T *a, int64_t a0, const T *b, int64_t b0, size_t n,
-                                                            size_t head, size_t nchunks, MapDev m,
-                                                            typename P::Part *__restrict__ partials)
+                                                            MapDev m, T init, int has_init, T *out, double *out_f64,
+                                                            Ctrl *ctrl, uint64_t *status, uint32_t ep)
 {
     using S = typename P::State;
     __shared__ S s_buf[kRedThreads];
     const T c = map_bits<T>(m.c);
     S acc;
     switch (m.fn) {
-    case BCMI_MAP_ABS: acc = fold_any<T, P, VEC, OPB, BCMI_MAP_ABS>(a, a0, b, b0, n, head, nchunks, c); break;
-    case BCMI_MAP_SQUARE: acc = fold_any<T, P, VEC, OPB, BCMI_MAP_SQUARE>(a, a0, b, b0, n, head, nchunks, c); break;
-    default: acc = fold_any<T, P, VEC, OPB, BCMI_MAP_ID>(a, a0, b, b0, n, head, nchunks, c); break;
+    case BCMI_MAP_ABS: acc = fold_any<T, P, VEC, OPB, BCMI_MAP_ABS>(a, a0, b, b0, n, c); break;
+    case BCMI_MAP_SQUARE: acc = fold_any<T, P, VEC, OPB, BCMI_MAP_SQUARE>(a, a0, b, b0, n, c); break;
+    default: acc = fold_any<T, P, VEC, OPB, BCMI_MAP_ID>(a, a0, b, b0, n, c); break;
     }
-    S blk = block_combine<S, P>(acc, s_buf);
-    if (threadIdx.x == 0) partials[blockIdx.x] = P::part(blk);
+    reduce_finish<T, P>(block_combine<S, P>(acc, s_buf), init, has_init, out, out_f64, ctrl, status,
+                        launch_epoch(ctrl, ep));
 }
 
 template <typename T, typename P, int OPB>
@@ -150,45 +145,29 @@ static int launch_mapreduce(bcmi_queue q, const bcmi_seq *a, const bcmi_seq *b, 
     const T *pa = (const T *)a->ptr;
     constexpr bool BIN = OPB != kMapUnary;
     const T *pb = BIN ? (const T *)b->ptr : nullptr;
-    // the chunked path needs arrays at one offset inside a 16-byte chunk;
-    // 8- and 16-bit elements always go element by element (the compiler's
-    // vectoriser fails on the 16-wide byte chunks of some maps)
-    const uintptr_t ma = (uintptr_t)pa & 15, mb = BIN ? ((uintptr_t)pb & 15) : ma;
-    const bool vec = sizeof(T) >= 4 && pa && (!BIN || pb) && ma == mb && ma % sizeof(T) == 0;
-    size_t head = 0, nchunks = 0;
-    if (vec) {
-        head = ma ? (16 - ma) / sizeof(T) : 0;
-        if (head > n) head = n;
-        nchunks = (n - head) / chunk16<T>::N;
-    }
-    const size_t work = vec ? nchunks : (n + 3) / 4;
-    const size_t want = (work + kRedThreads * 8 - 1) / (kRedThreads * 8);
-    const size_t maxb = (size_t)q->cu_count * 4;
-    const size_t blocks = want < 1 ? 1 : (want > maxb ? maxb : want);
-    void *scr;
-    BCMI_TRY(scratch(q, blocks * sizeof(typename P::Part), &scr));
+    // the chunked path needs arrays of 4- or 8-byte elements; 8- and 16-bit
+    // elements always go element by element (the compiler's vectoriser fails
+    // on the 16-wide byte chunks of some maps)
+    const bool vec = sizeof(T) >= 4 && pa && (!BIN || pb);
+    const unsigned blocks = reduce_blocks(q, vec ? n / chunk16<T>::N : (n + 3) / 4, 4);
+    uint64_t *status;
+    BCMI_TRY(status_array(q, (size_t)blocks * kPartWords, &status));
+    Epochs ep;
+    BCMI_TRY(begin_lookback(q, 1, &ep));
     T ini{};
     if (init) memcpy(&ini, init, sizeof(T));
     const int64_t a0 = a->start, b0 = BIN ? b->start : 0;
-    if constexpr (sizeof(T) >= 4) {
-        if (vec) {
-            BCMI_LAUNCH(q, "mapreduce",
-                        hipLaunchKernelGGL((k_mapreduce<T, P, true, OPB>), dim3((unsigned)blocks), dim3(kRedThreads),
-                                           0, q->stream, pa, a0, pb, b0, n, head, nchunks, m,
-                                           (typename P::Part *)scr));
-        }
-    }
-    if (!vec) {
+    auto go = [&](auto v) {
         BCMI_LAUNCH(q, "mapreduce",
-                    hipLaunchKernelGGL((k_mapreduce<T, P, false, OPB>), dim3((unsigned)blocks), dim3(kRedThreads), 0,
-                                       q->stream, pa, a0, pb, b0, n, head, nchunks, m,
-                                       (typename P::Part *)scr));
+                    hipLaunchKernelGGL((k_mapreduce<T, P, decltype(v)::value, OPB>), dim3(blocks), dim3(kRedThreads),
+                                       0, q->stream, pa, a0, pb, b0, n, m, ini, init ? 1 : 0, (T *)out, out_f64,
+                                       q->ctrl, status, ep.arg(0)));
+        return 0;
+    };
+    if constexpr (sizeof(T) >= 4) {
+        if (vec) return go(std::true_type());
     }
-    BCMI_LAUNCH(q, "mapreduce_final",
-                hipLaunchKernelGGL((k_reduce_final<T, P>), dim3(1), dim3(kRedThreads), 0, q->stream,
-                                   (const typename P::Part *)scr, (uint32_t)blocks, ini, init ? 1 : 0, (T *)out,
-                                   out_f64));
-    return 0;
+    return go(std::false_type());
 }
 
 template <typename T, typename P>

@@ -8,9 +8,9 @@
 //
 // Here: one launch.  A grid of a few blocks per CU streams the input with
 // 128-bit loads; each thread keeps a compensated FP32 pair (TwoSum) for
-// float plus, waves combine pairs with DPP, the block writes one FP64
-// partial, and a one-block kernel folds the partials in FP64 in a fixed
-// order (so the result is deterministic).  Integers wrap exactly;
+// float plus, waves combine pairs with DPP, the block publishes one FP64
+// partial, and the last block folds the partials in FP64 in a fixed order
+// (so the result is deterministic).  Integers wrap exactly;
 // min/max/multiplies fold in the element type.
 #include "reduce.hpp"
 
@@ -22,20 +22,19 @@ namespace bcmi {
 
 // U chunks of 16 bytes in flight per thread and iteration.
 template <typename T, typename P, int U>
-__global__ __launch_bounds__(kRedThreads) void k_reduce(const T *__restrict__ in, size_t n, size_t head,
-                                                        size_t nchunks, typename P::Part *__restrict__ partials)
+__global__ __launch_bounds__(kRedThreads) void k_reduce(const T *__restrict__ in, size_t n, T init, int has_init,
+                                                        T *out, double *out_f64, Ctrl *ctrl, uint64_t *status,
+                                                        uint32_t ep)
 {
     using S = typename P::State;
     __shared__ S s_buf[kRedThreads];
 
     S acc = P::id();
-    // head/tail elements outside the aligned 16-byte body: block 0
-    const size_t tail0 = head + nchunks * chunk16<T>::N;
-    if (blockIdx.x == 0) {
-        for (size_t i = threadIdx.x; i < head; i += kRedThreads) acc = P::add(acc, in[i]);
-        for (size_t i = tail0 + threadIdx.x; i < n; i += kRedThreads) acc = P::add(acc, in[i]);
-    }
-    const chunk16<T> *body = (const chunk16<T> *)(in + head);
+    const size_t nchunks = n / chunk16<T>::N;
+    // elements after the last whole chunk: block 0
+    if (blockIdx.x == 0)
+        for (size_t i = nchunks * chunk16<T>::N + threadIdx.x; i < n; i += kRedThreads) acc = P::add(acc, in[i]);
+    const chunk16<T> *body = (const chunk16<T> *)in;
     const size_t stride = (size_t)gridDim.x * kRedThreads;
     size_t c = (size_t)blockIdx.x * kRedThreads + threadIdx.x;
     for (; c + (U - 1) * stride < nchunks; c += U * stride) {
@@ -52,47 +51,35 @@ __global__ __launch_bounds__(kRedThreads) void k_reduce(const T *__restrict__ in
 #pragma unroll
         for (int k = 0; k < chunk16<T>::N; ++k) acc = P::add(acc, a.v[k]);
     }
-    S blk = block_combine<S, P>(acc, s_buf);
-    if (threadIdx.x == 0) partials[blockIdx.x] = P::part(blk);
+    reduce_finish<T, P>(block_combine<S, P>(acc, s_buf), init, has_init, out, out_f64, ctrl, status,
+                        launch_epoch(ctrl, ep));
 }
 
 template <typename T, typename P>
 static int run_reduce(bcmi_queue q, const void *in_, size_t n, const void *init, void *out, double *out_f64)
 {
     const T *in = (const T *)in_;
-    size_t head = 0;
-    uintptr_t mis = (uintptr_t)in & 15;
-    if (mis) {
-        if (mis % sizeof(T)) head = n;  // not element-aligned to a chunk: scalar only
-        else head = (16 - mis) / sizeof(T);
-    }
-    if (head > n) head = n;
-    size_t nchunks = (n - head) / chunk16<T>::N;
     // chunks in flight per thread ("unroll": 2, 4 or 8) and workgroups per
     // CU ("blocks_per_cu") come from the tuning cache (key "__bcmi_reduce")
     const unsigned unroll = tune_get("__bcmi_reduce", "unroll", 2);
     const unsigned bpc = tune_get("__bcmi_reduce", "blocks_per_cu", 4);
-    size_t want = (nchunks + kRedThreads * 8 - 1) / (kRedThreads * 8);
-    size_t maxb = (size_t)q->cu_count * (bpc ? bpc : 4);
-    size_t blocks = want < 1 ? 1 : (want > maxb ? maxb : want);
-    void *scr;
-    BCMI_TRY(scratch(q, blocks * sizeof(typename P::Part), &scr));
+    const unsigned blocks = reduce_blocks(q, n / chunk16<T>::N, bpc && bpc <= kPartBlocksPerCU ? bpc : 4);
+    uint64_t *status;
+    BCMI_TRY(status_array(q, (size_t)blocks * kPartWords, &status));
+    Epochs ep;
+    BCMI_TRY(begin_lookback(q, 1, &ep));
     T ini{};
     if (init) memcpy(&ini, init, sizeof(T));
     auto go = [&](auto u) {
         BCMI_LAUNCH(q, "reduce",
-                    hipLaunchKernelGGL((k_reduce<T, P, decltype(u)::value>), dim3((unsigned)blocks), dim3(kRedThreads),
-                                       0, q->stream, in, n, head, nchunks, (typename P::Part *)scr));
+                    hipLaunchKernelGGL((k_reduce<T, P, decltype(u)::value>), dim3(blocks), dim3(kRedThreads), 0,
+                                       q->stream, in, n, ini, init ? 1 : 0, (T *)out, out_f64, q->ctrl, status,
+                                       ep.arg(0)));
         return 0;
     };
-    if (unroll >= 8) BCMI_TRY(go(std::integral_constant<int, 8>()));
-    else if (unroll >= 4) BCMI_TRY(go(std::integral_constant<int, 4>()));
-    else BCMI_TRY(go(std::integral_constant<int, 2>()));
-    BCMI_LAUNCH(q, "reduce_final",
-                hipLaunchKernelGGL((k_reduce_final<T, P>), dim3(1), dim3(kRedThreads), 0, q->stream,
-                                   (const typename P::Part *)scr, (uint32_t)blocks, ini, init ? 1 : 0, (T *)out,
-                                   out_f64));
-    return 0;
+    if (unroll >= 8) return go(std::integral_constant<int, 8>());
+    if (unroll >= 4) return go(std::integral_constant<int, 4>());
+    return go(std::integral_constant<int, 2>());
 }
 
 template <typename T>

@@ -106,9 +106,10 @@ struct CompF64Policy {
     static BDEV double f64(Part p) { return p.s + p.c; }
 };
 
-// 16-byte-chunk view of the input
+// 16-byte-chunk view of the input, aligned as its elements are (a
+// buffer_iterator may start anywhere)
 template <typename T>
-struct alignas(16) chunk16 {
+struct chunk16 {
     static constexpr int N = 16 / sizeof(T);
     T v[N];
 };
@@ -140,28 +141,80 @@ BDEV S block_combine(S v, S *s_buf)
     }
 }
 
-// One block folds the per-block partials in FP64 / the element type in a
-// fixed order, so the result is deterministic.
+// A block's partial as tagged status words (device.hpp): 32 bits of it each.
+template <typename Pt>
+struct PartBox {
+    static constexpr int N = (int)(sizeof(Pt) + 3) / 4;
+    static_assert(N <= kPartWords, "partial of at most kPartWords words");
+    uint32_t w[N];
+};
+
+template <typename Pt>
+BDEV void part_publish(uint64_t *status, uint32_t block, uint32_t epoch, Pt p)
+{
+    PartBox<Pt> b{};
+    __builtin_memcpy(b.w, &p, sizeof(Pt));
+    lb_publish(status, block, epoch, LB_A, b);
+}
+
+// A bounded wait (every block but the last publishes without waiting, and
+// blocks are dispatched in order, so it ends).
+template <typename Pt>
+BDEV Pt part_wait(const uint64_t *status, uint32_t block, uint32_t epoch, Ctrl *ctrl)
+{
+    PartBox<Pt> b{};
+    uint32_t spins = 0;
+    while (lb_read(status, block, epoch, b) == LB_X)
+        if (spin_expired(ctrl, spins)) break;
+    Pt p;
+    __builtin_memcpy(&p, b.w, sizeof(Pt));
+    return p;
+}
+
+// Called by all threads of every block with the block's folded state.  The
+// last block folds all blocks' partials in a fixed order (so the result is
+// deterministic) and finishes the result.  The partials come through the
+// tagged status words rather than through a second launch of one block: that
+// kernel took 2.5 us behind a first one of 3.3 us at 65,537 floats, and the
+// words carry their own arrival, so no fence or device-scope atomic is needed.
 template <typename T, typename P>
-__global__ __launch_bounds__(kRedThreads) void k_reduce_final(const typename P::Part *__restrict__ partials,
-                                                              uint32_t nparts, T init, int has_init, T *out,
-                                                              double *out_f64)
+BDEV void reduce_finish(typename P::State blk, T init, int has_init, T *out, double *out_f64, Ctrl *ctrl,
+                        uint64_t *status, uint32_t epoch)
 {
     using Pt = typename P::Part;
-    __shared__ Pt s_part[kRedThreads];
-    Pt p = P::part_id();
-    for (uint32_t i = threadIdx.x; i < nparts; i += kRedThreads) p = P::part_merge(p, partials[i]);
-    s_part[threadIdx.x] = p;
-    block_barrier();
-    for (int off = kRedThreads / 2; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) s_part[threadIdx.x] = P::part_merge(s_part[threadIdx.x], s_part[threadIdx.x + off]);
+    const uint32_t last = gridDim.x - 1;
+    Pt total = P::part(blk);
+    if (blockIdx.x != last) {
+        if (threadIdx.x == 0) part_publish<Pt>(status, blockIdx.x, epoch, total);
+        return;
+    }
+    if (last > 0) {
+        __shared__ Pt s_part[kRedThreads];
+        Pt p = P::part_id();
+        for (uint32_t i = threadIdx.x; i <= last; i += kRedThreads)
+            p = P::part_merge(p, i == last ? total : part_wait<Pt>(status, i, epoch, ctrl));
+        s_part[threadIdx.x] = p;
         block_barrier();
+        for (int off = kRedThreads / 2; off > 0; off >>= 1) {
+            if ((int)threadIdx.x < off)
+                s_part[threadIdx.x] = P::part_merge(s_part[threadIdx.x], s_part[threadIdx.x + off]);
+            block_barrier();
+        }
+        total = s_part[0];
     }
     if (threadIdx.x == 0) {
-        Pt total = s_part[0];
         *out = P::finish(total, has_init != 0, init);
         if (out_f64) *out_f64 = P::f64(total) + (has_init ? (double)init : 0.0);
     }
+}
+
+// Blocks of a streaming reduction over `chunks` 16-byte chunks: two chunks a
+// thread (one load round trip) until the grid holds per_cu blocks per CU.
+inline unsigned reduce_blocks(bcmi_queue q, size_t chunks, unsigned per_cu)
+{
+    const size_t want = (chunks + kRedThreads * 2 - 1) / (kRedThreads * 2);
+    const size_t most = (size_t)q->cu_count * per_cu;
+    return (unsigned)(want < 1 ? 1 : (want > most ? most : want));
 }
 
 }  // namespace bcmi

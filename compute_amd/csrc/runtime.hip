@@ -282,6 +282,14 @@ int bcmi_queue_create(int device, bcmi_queue *queue)
         bcmi_queue_destroy(q);
         return s;
     }
+    // the words that the reductions' block partials need at most, so that
+    // they never grow the array (a capture may be a queue's first call)
+    uint64_t *words;
+    const int st = status_array(q, (size_t)q->cu_count * kPartBlocksPerCU * kPartWords, &words);
+    if (st) {
+        bcmi_queue_destroy(q);
+        return st;
+    }
     *queue = q;
     return 0;
 }

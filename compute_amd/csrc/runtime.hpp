@@ -63,6 +63,11 @@ struct Epochs {
     }
 };
 
+// Block partials of a reduction handed over in the status array: at most
+// kPartBlocksPerCU blocks per CU, kPartWords words each.
+constexpr int kPartBlocksPerCU = 8;
+constexpr int kPartWords = 4;
+
 struct ProfRec {
     const char *name;
     hipEvent_t start, stop;
