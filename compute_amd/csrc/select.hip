@@ -20,7 +20,7 @@
 // as the reference's scan-based scatter gives.  Tiles are laid over the
 // 16-byte-aligned address space: positions before `in` (a buffer_iterator
 // offset) are masked off, so every full chunk is one 16-byte load.
-#include "device.hpp"
+#include "reduce.hpp"
 
 #include <algorithm>
 #include <cstring>
@@ -144,12 +144,13 @@ enum : int {
 #define BCMI_SEL_STAGE 32768  // LDS bytes of output staging per block
 #endif
 
-template <typename T>
+// DIV: 1, or 4 for ranges that would leave most of the chip without a tile.
+template <typename T, int DIV = 1>
 struct SelShape {
-    static constexpr int V = 16 / (int)sizeof(T);                               // elements per chunk
-    static constexpr int EPT = sizeof(T) == 8 ? BCMI_SEL_EPT8 : BCMI_SEL_EPT4;  // one flag word per thread
-    static constexpr int Q = EPT / V;                                           // chunks per thread
-    static constexpr int WSEG = Q * 64 * V;                                     // elements per wave
+    static constexpr int V = 16 / (int)sizeof(T);                                       // elements per chunk
+    static constexpr int EPT = (sizeof(T) == 8 ? BCMI_SEL_EPT8 : BCMI_SEL_EPT4) / DIV;  // one flag word per thread
+    static constexpr int Q = EPT / V;                                                   // chunks per thread
+    static constexpr int WSEG = Q * 64 * V;                                             // elements per wave
     static constexpr int TILE = 4 * WSEG;
     using F = std::conditional_t<(EPT > 32), uint64_t, uint32_t>;  // flag word
 };
@@ -158,12 +159,12 @@ struct SelShape {
 // each, so the staging buffer stays within BCMI_SEL_STAGE bytes.  Index
 // modes stage the position inside the tile (the index is formed when it is
 // written).
-template <typename T, int MODE>
+template <typename T, int MODE, int DIV>
 struct SelLds {
     using S = std::conditional_t<MODE == kSelIdx32 || MODE == kSelIdx64, uint32_t, T>;
-    static constexpr size_t BYTES = (size_t)SelShape<T>::TILE * sizeof(S);
+    static constexpr size_t BYTES = (size_t)SelShape<T, DIV>::TILE * sizeof(S);
     static constexpr int ROUNDS = BYTES > 2 * BCMI_SEL_STAGE ? 4 : BYTES > BCMI_SEL_STAGE ? 2 : 1;
-    S stage[SelShape<T>::TILE / ROUNDS];
+    S stage[SelShape<T, DIV>::TILE / ROUNDS];
     uint32_t wcnt[4];
     uint32_t prefix;
     uint32_t bad;
@@ -176,11 +177,9 @@ struct alignas(16) sel_chunk {
 
 // Flags of the elements (bit q*V + k for chunk q, element k) under the
 // predicate FN; invalid elements get 0.
-template <typename T, int FN, typename OK>
-BDEV typename SelShape<T>::F sel_flags(const T (&x)[SelShape<T>::Q][SelShape<T>::V], const SelPred &p, OK ok)
+template <typename F, typename T, int FN, int Q, int V, typename OK>
+BDEV F sel_flags(const T (&x)[Q][V], const SelPred &p, OK ok)
 {
-    using F = typename SelShape<T>::F;
-    constexpr int V = SelShape<T>::V, Q = SelShape<T>::Q;
     F f = 0;
 #pragma unroll
     for (int q = 0; q < Q; ++q)
@@ -190,15 +189,15 @@ BDEV typename SelShape<T>::F sel_flags(const T (&x)[SelShape<T>::Q][SelShape<T>:
     return f;
 }
 
-template <typename T, int MODE, bool FULL>
-BDEV void select_body(SelLds<T, MODE> &L, const T *abase, size_t head, size_t n, void *out_a, void *out_b,
+template <typename T, int MODE, int DIV, bool FULL>
+BDEV void select_body(SelLds<T, MODE, DIV> &L, const T *abase, size_t head, size_t n, void *out_a, void *out_b,
                       const SelPred &p, Ctrl *ctrl, uint64_t *status, uint64_t *count_out, uint32_t epoch)
 {
-    using Sh = SelShape<T>;
+    using Sh = SelShape<T, DIV>;
     using C = typename SelCmp<T>::type;
     using F = typename Sh::F;
     constexpr int V = Sh::V, Q = Sh::Q, WSEG = Sh::WSEG, TILE = Sh::TILE;
-    constexpr int ROUNDS = SelLds<T, MODE>::ROUNDS, WPR = 4 / ROUNDS, RSEG = WPR * WSEG;
+    constexpr int ROUNDS = SelLds<T, MODE, DIV>::ROUNDS, WPR = 4 / ROUNDS, RSEG = WPR * WSEG;
 
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const uint32_t tile = blockIdx.x;
@@ -257,16 +256,16 @@ BDEV void select_body(SelLds<T, MODE> &L, const T *abase, size_t head, size_t n,
         }
     } else if constexpr (std::is_floating_point<T>::value) {
         switch (p.fn) {
-        case BCMI_FN_MUL: f = sel_flags<T, BCMI_FN_MUL>(x, p, ok); break;
-        case BCMI_FN_SIGNBIT: f = sel_flags<T, BCMI_FN_SIGNBIT>(x, p, ok); break;
-        default: f = sel_flags<T, BCMI_FN_ID>(x, p, ok); break;
+        case BCMI_FN_MUL: f = sel_flags<F, T, BCMI_FN_MUL>(x, p, ok); break;
+        case BCMI_FN_SIGNBIT: f = sel_flags<F, T, BCMI_FN_SIGNBIT>(x, p, ok); break;
+        default: f = sel_flags<F, T, BCMI_FN_ID>(x, p, ok); break;
         }
     } else {
         switch (p.fn) {
-        case BCMI_FN_MUL: f = sel_flags<T, BCMI_FN_MUL>(x, p, ok); break;
-        case BCMI_FN_MOD: f = sel_flags<T, BCMI_FN_MOD>(x, p, ok); break;
-        case BCMI_FN_AND: f = sel_flags<T, BCMI_FN_AND>(x, p, ok); break;
-        default: f = sel_flags<T, BCMI_FN_ID>(x, p, ok); break;
+        case BCMI_FN_MUL: f = sel_flags<F, T, BCMI_FN_MUL>(x, p, ok); break;
+        case BCMI_FN_MOD: f = sel_flags<F, T, BCMI_FN_MOD>(x, p, ok); break;
+        case BCMI_FN_AND: f = sel_flags<F, T, BCMI_FN_AND>(x, p, ok); break;
+        default: f = sel_flags<F, T, BCMI_FN_ID>(x, p, ok); break;
         }
     }
 
@@ -376,19 +375,19 @@ BDEV void select_body(SelLds<T, MODE> &L, const T *abase, size_t head, size_t n,
 #define BCMI_SEL_WPE 4  // minimum waves per SIMD the register allocation must allow
 #endif
 
-template <typename T, int MODE>
-__global__ __launch_bounds__(kSelThreads) __attribute__((amdgpu_waves_per_eu(BCMI_SEL_WPE))) void k_select(const T *abase, size_t head, size_t n, void *out_a,
-                                                        void *out_b, SelPred p, Ctrl *ctrl, uint64_t *status,
-                                                        uint64_t *count_out, uint32_t back)
+template <typename T, int MODE, int DIV>
+__global__ __launch_bounds__(kSelThreads) __attribute__((amdgpu_waves_per_eu(BCMI_SEL_WPE))) void k_select(
+    const T *abase, size_t head, size_t n, void *out_a, void *out_b, SelPred p, Ctrl *ctrl, uint64_t *status,
+    uint64_t *count_out, uint32_t back)
 {
-    constexpr size_t TILE = SelShape<T>::TILE;
-    __shared__ SelLds<T, MODE> lds;
+    constexpr size_t TILE = SelShape<T, DIV>::TILE;
+    __shared__ SelLds<T, MODE, DIV> lds;
     const size_t tstart = (size_t)blockIdx.x * TILE;
     const uint32_t epoch = launch_epoch(ctrl, back);
     if (tstart >= head && tstart + TILE <= head + n)
-        select_body<T, MODE, true>(lds, abase, head, n, out_a, out_b, p, ctrl, status, count_out, epoch);
+        select_body<T, MODE, DIV, true>(lds, abase, head, n, out_a, out_b, p, ctrl, status, count_out, epoch);
     else
-        select_body<T, MODE, false>(lds, abase, head, n, out_a, out_b, p, ctrl, status, count_out, epoch);
+        select_body<T, MODE, DIV, false>(lds, abase, head, n, out_a, out_b, p, ctrl, status, count_out, epoch);
 }
 
 // stable_partition, pass 2: out[i] = tmp[i] below the selected count, and
@@ -408,8 +407,8 @@ __global__ void k_set_count(uint64_t *count, uint64_t v)
     if (threadIdx.x == 0) *count = v;
 }
 
-// count_if: a grid of a few blocks per CU streams 16-byte chunks; block
-// partials, then one block sums them in a fixed order.
+// count_if: a grid of a few blocks per CU streams 16-byte chunks; the last
+// block adds up the blocks' counts.
 template <typename T, int FN>
 BDEV uint32_t count_range(const T *in, size_t head, size_t n, size_t nchunks, const SelPred &p)
 {
@@ -438,7 +437,8 @@ BDEV uint32_t count_range(const T *in, size_t head, size_t n, size_t nchunks, co
 
 template <typename T>
 __global__ __launch_bounds__(kSelThreads) void k_count_if(const T *in, size_t head, size_t n, size_t nchunks,
-                                                          SelPred p, uint64_t *partials)
+                                                          SelPred p, uint64_t *count, Ctrl *ctrl, uint64_t *status,
+                                                          uint32_t ep)
 {
     __shared__ uint32_t s_w[kSelThreads / 64];
     uint32_t c;
@@ -459,22 +459,21 @@ __global__ __launch_bounds__(kSelThreads) void k_count_if(const T *in, size_t he
     c = wave_reduce(c, 0u, [](uint32_t a, uint32_t b) { return a + b; });
     if ((threadIdx.x & 63) == 0) s_w[threadIdx.x >> 6] = c;
     block_barrier();
-    if (threadIdx.x == 0) partials[blockIdx.x] = (uint64_t)s_w[0] + s_w[1] + s_w[2] + s_w[3];
-}
-
-__global__ __launch_bounds__(kSelThreads) void k_count_final(const uint64_t *partials, uint32_t nparts,
-                                                             uint64_t *count)
-{
-    __shared__ uint64_t s[kSelThreads];
-    uint64_t c = 0;
-    for (uint32_t i = threadIdx.x; i < nparts; i += kSelThreads) c += partials[i];
-    s[threadIdx.x] = c;
-    block_barrier();
-    for (int off = kSelThreads / 2; off > 0; off >>= 1) {
-        if ((int)threadIdx.x < off) s[threadIdx.x] += s[threadIdx.x + off];
-        block_barrier();
+    // the last block adds up the others' counts (reduce_finish in reduce.hpp:
+    // tagged words instead of a second launch)
+    const uint64_t own = (uint64_t)s_w[0] + s_w[1] + s_w[2] + s_w[3];
+    const uint32_t last = gridDim.x - 1, epoch = launch_epoch(ctrl, ep);
+    if (blockIdx.x != last) {
+        if (threadIdx.x == 0) part_publish<uint64_t>(status, blockIdx.x, epoch, own);
+        return;
     }
-    if (threadIdx.x == 0) *count = s[0];
+    uint64_t t = threadIdx.x == 0 ? own : 0;
+    for (uint32_t i = threadIdx.x; i < last; i += kSelThreads) t += part_wait<uint64_t>(status, i, epoch, ctrl);
+    __shared__ uint64_t s_t[kSelThreads / 64];
+    t = wave_reduce(t, (uint64_t)0, [](uint64_t a, uint64_t b) { return a + b; });
+    if ((threadIdx.x & 63) == 0) s_t[threadIdx.x >> 6] = t;
+    block_barrier();
+    if (threadIdx.x == 0) *count = s_t[0] + s_t[1] + s_t[2] + s_t[3];
 }
 
 // ---------------------------------------------------------------- host side
@@ -522,13 +521,12 @@ static int make_pred(int dtype, const bcmi_predicate *pr, SelPred *p)
     return 0;
 }
 
-template <typename T, int MODE>
-static int launch_select(bcmi_queue q, const T *in, void *out_a, void *out_b, size_t n, const SelPred &p,
-                         uint64_t *count_out)
+template <typename T, int MODE, int DIV>
+static int launch_select_div(bcmi_queue q, const T *in, void *out_a, void *out_b, size_t n, const SelPred &p,
+                             uint64_t *count_out)
 {
-    constexpr size_t TILE = SelShape<T>::TILE;
+    constexpr size_t TILE = SelShape<T, DIV>::TILE;
     const size_t head = ((uintptr_t)in & 15) / sizeof(T);
-    BCMI_CHECK(((uintptr_t)in % sizeof(T)) == 0, BCMI_INVALID_VALUE, "select: input not element-aligned");
     const T *abase = in - head;
     const size_t tiles = (n + head + TILE - 1) / TILE;
     BCMI_CHECK(tiles < (1ull << 31), BCMI_INVALID_BUFFER_SIZE, "select: n=%zu too large", n);
@@ -537,9 +535,24 @@ static int launch_select(bcmi_queue q, const T *in, void *out_a, void *out_b, si
     Epochs ep;
     BCMI_TRY(begin_lookback(q, 1, &ep));
     BCMI_LAUNCH(q, "select",
-                hipLaunchKernelGGL((k_select<T, MODE>), dim3((unsigned)tiles), dim3(kSelThreads), 0, q->stream,
+                hipLaunchKernelGGL((k_select<T, MODE, DIV>), dim3((unsigned)tiles), dim3(kSelThreads), 0, q->stream,
                                    abase, head, n, out_a, out_b, p, q->ctrl, status, count_out, ep.arg(0)));
     return 0;
+}
+
+template <typename T, int MODE>
+static int launch_select(bcmi_queue q, const T *in, void *out_a, void *out_b, size_t n, const SelPred &p,
+                         uint64_t *count_out)
+{
+    BCMI_CHECK(((uintptr_t)in % sizeof(T)) == 0, BCMI_INVALID_VALUE, "select: input not element-aligned");
+    // Tiles of a quarter of the elements until the full ones would number a
+    // few hundred: one tile per CU leaves its loads, ranks and stores in
+    // series.  us a call, quarter tiles first: copy_if of int32 1 M: 6.5 11.3,
+    // 4 M: 12.0 14.9, 8 M: 19.6 19.0; of int64 1 M: 8.2 9.2, 2 M: 11.2 11.1;
+    // partition_copy of int32 4 M: 14.4 17.0, 8 M: 22.9 22.4.
+    if (n <= (size_t)SelShape<T>::TILE * (sizeof(T) == 8 ? 192 : 384))
+        return launch_select_div<T, MODE, 4>(q, in, out_a, out_b, n, p, count_out);
+    return launch_select_div<T, MODE, 1>(q, in, out_a, out_b, n, p, count_out);
 }
 
 template <typename T>
@@ -588,17 +601,14 @@ static int run_count_if(bcmi_queue q, const void *in_, size_t n, const SelPred &
     if (mis) head = (mis % sizeof(T)) ? n : (16 - mis) / sizeof(T);
     if (head > n) head = n;
     const size_t nchunks = (n - head) / V;
-    const size_t want = (nchunks + kSelThreads - 1) / kSelThreads;
-    const unsigned blocks = (unsigned)std::max<size_t>(1, std::min<size_t>(want, (size_t)cu_blocks(q, 4)));
-    void *sp;
-    BCMI_TRY(scratch(q, blocks * sizeof(uint64_t), &sp));
-    uint64_t *partials = (uint64_t *)sp;
+    const unsigned blocks = reduce_blocks(q, nchunks, 4);
+    uint64_t *status;
+    BCMI_TRY(status_array(q, (size_t)blocks * kPartWords, &status));
+    Epochs ep;
+    BCMI_TRY(begin_lookback(q, 1, &ep));
     BCMI_LAUNCH(q, "count_if",
                 hipLaunchKernelGGL((k_count_if<T>), dim3(blocks), dim3(kSelThreads), 0, q->stream, in, head, n,
-                                   nchunks, p, partials));
-    BCMI_LAUNCH(q, "count_final",
-                hipLaunchKernelGGL(k_count_final, dim3(1), dim3(kSelThreads), 0, q->stream, (const uint64_t *)partials,
-                                   blocks, count));
+                                   nchunks, p, count, q->ctrl, status, ep.arg(0)));
     return 0;
 }
 
