@@ -96,8 +96,11 @@ struct ArraySrc {
     BDEV T map(T x) const { return x; }
 };
 
+// 16 bytes of elements, aligned as the elements are: a range may start
+// anywhere in its allocation, and a wave's chunks are one contiguous 1 KB
+// whether or not it lies on the 16-byte grid.
 template <typename T>
-struct alignas(16) sc_chunk {
+struct sc_chunk {
     static constexpr int N = 16 / sizeof(T);
     T v[N];
 };
@@ -194,15 +197,14 @@ BDEV void chunks_from_rows(const T (&b)[Q * 4], T (&s)[Q][4], uint32_t *buf, uin
 // One tile: Q 16-byte chunks per thread (tile = NW waves * 64 lanes * Q
 // chunks), wave-striped: chunk q of lane l of wave w covers elements
 // w*WSEG + q*64*V + l*V .. +V-1 of the tile.  FULL: the tile lies below n, so
-// no element needs a bounds test.  VEC: input and output are 16-byte
-// aligned, so full chunks move as one 16-byte load / store.  BG > 0 (4-byte
-// elements): the loaded chunks are transposed, BG chunks at a time, into
+// no element needs a bounds test and every chunk moves as one 16-byte load
+// or store.  BG > 0 (4-byte elements): the loaded chunks are transposed, BG chunks at a time, into
 // blocked rows through the wave's LDS buffer (blk, RowShape<Q, BG>::WORDS
 // words per wave) so that each lane scans Q*4 consecutive elements serially
 // and the wave scans one fold per lane instead of one per chunk; the
 // results go back to striped chunks the same way.  That trades Q wave
 // scans per tile for two LDS round trips.
-template <typename T, typename P, bool VEC, int Q, int NW, bool FULL, int BG, typename Src>
+template <typename T, typename P, int Q, int NW, bool FULL, int BG, typename Src>
 BDEV void scan_body(ScanLds<P, NW> &L, uint32_t *blk, const Src src, T *out, size_t n, Ctrl *ctrl,
                     uint64_t *status, typename P::Cr init, int exclusive, uint32_t epoch)
 {
@@ -223,6 +225,9 @@ BDEV void scan_body(ScanLds<P, NW> &L, uint32_t *blk, const Src src, T *out, siz
     // blocked position e of this lane (BLK)
     auto okb = [&](int e) { return FULL || (int64_t)(lane * Q * V + e) < rem; };
     constexpr bool BLK = BG > 0;
+    // the last tile's whole chunks move as vectors too, where that costs no
+    // spills (the shapes that small ranges take)
+    constexpr bool PV = Q <= 4;
     uint32_t *wblk = blk + w * RowShape<Q, BLK ? BG : Q>::WORDS;
 
     T x[Q][V];
@@ -230,7 +235,7 @@ BDEV void scan_body(ScanLds<P, NW> &L, uint32_t *blk, const Src src, T *out, siz
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             const T *p = win + q * 64 * V + lane * V;
-            if (VEC && FULL) {
+            if (FULL || (PV && ok(q, V - 1))) {
                 const sc_chunk<T> c = *(const sc_chunk<T> *)p;
 #pragma unroll
                 for (int k = 0; k < V; ++k) x[q][k] = src.map(c.v[k]);
@@ -314,7 +319,7 @@ BDEV void scan_body(ScanLds<P, NW> &L, uint32_t *blk, const Src src, T *out, siz
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             T *dst = wout + q * 64 * V + lane * V;
-            if (VEC && FULL) {
+            if (FULL || (PV && ok(q, V - 1))) {
                 sc_chunk<T> c;
 #pragma unroll
                 for (int k = 0; k < V; ++k) c.v[k] = x[q][k];
@@ -346,7 +351,7 @@ BDEV void scan_body(ScanLds<P, NW> &L, uint32_t *blk, const Src src, T *out, siz
             y[k] = P::out(prefix, exclusive ? before : s);
         }
         T *dst = wout + q * 64 * V + lane * V;
-        if (VEC && FULL) {
+        if (FULL || (PV && ok(q, V - 1))) {
             sc_chunk<T> c;
 #pragma unroll
             for (int k = 0; k < V; ++k) c.v[k] = y[k];
@@ -362,7 +367,7 @@ BDEV void scan_body(ScanLds<P, NW> &L, uint32_t *blk, const Src src, T *out, siz
 // NW waves per workgroup (4, or 8: a tile twice as big, half the tiles and
 // look-backs).
 // WPE: waves per SIMD the register allocation must allow (1: no bound).
-template <typename T, typename P, bool VEC, int Q, typename Src, int NW = 4, int BG = 0, int WPE = 1>
+template <typename T, typename P, int Q, typename Src, int NW = 4, int BG = 0, int WPE = 1>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE))) void k_scan(
     const Src src, T *out, size_t n, Ctrl *ctrl, uint64_t *status, typename P::Cr init, int exclusive,
     uint32_t back)
@@ -376,9 +381,9 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(WPE))) 
     }
     const uint32_t epoch = launch_epoch(ctrl, back);
     if ((size_t)(blockIdx.x + 1) * TILE <= n)
-        scan_body<T, P, VEC, Q, NW, true, BG>(lds, blk, src, out, n, ctrl, status, init, exclusive, epoch);
+        scan_body<T, P, Q, NW, true, BG>(lds, blk, src, out, n, ctrl, status, init, exclusive, epoch);
     else
-        scan_body<T, P, VEC, Q, NW, false, BG>(lds, blk, src, out, n, ctrl, status, init, exclusive, epoch);
+        scan_body<T, P, Q, NW, false, BG>(lds, blk, src, out, n, ctrl, status, init, exclusive, epoch);
 }
 
 template <typename T, typename P, int Q, typename Src, int NW = 4, int BG = 0, int WPE = 1>
@@ -388,29 +393,34 @@ static int launch_scan(bcmi_queue q, const Src &src, T *out, size_t n, uint64_t 
     constexpr size_t TILE = (size_t)NW * Q * 64 * (16 / sizeof(T));
     size_t tiles = (n + TILE - 1) / TILE;
     BCMI_CHECK(tiles < (1ull << 31), BCMI_INVALID_BUFFER_SIZE, "scan: n=%zu too large", n);
-    bool vec = (((uintptr_t)src.ptr | (uintptr_t)out) & 15) == 0;
     Epochs ep;
     BCMI_TRY(begin_lookback(q, 1, &ep));
-    if (vec) {
-        BCMI_LAUNCH(q, "scan",
-                    hipLaunchKernelGGL((k_scan<T, P, true, Q, Src, NW, BG, WPE>), dim3((unsigned)tiles), dim3(NW * 64), 0,
-                                       q->stream, src, out, n, q->ctrl, status, ini, exclusive, ep.arg(0)));
-    } else {
-        BCMI_LAUNCH(q, "scan",
-                    hipLaunchKernelGGL((k_scan<T, P, false, Q, Src, NW, BG, WPE>), dim3((unsigned)tiles), dim3(NW * 64), 0,
-                                       q->stream, src, out, n, q->ctrl, status, ini, exclusive, ep.arg(0)));
-    }
+    BCMI_LAUNCH(q, "scan",
+                hipLaunchKernelGGL((k_scan<T, P, Q, Src, NW, BG, WPE>), dim3((unsigned)tiles), dim3(NW * 64), 0,
+                                   q->stream, src, out, n, q->ctrl, status, ini, exclusive, ep.arg(0)));
     return 0;
 }
 
-// Chunks per thread come from the tuning cache (key "__bcmi_scan", or
-// "__bcmi_scan_f32" for the compensated float scan; param "q": 4, 8 or 16;
-// param "waves": 4, or 8 with q = 8 or 16) for 4-byte array scans; 4
-// chunks and 4 waves otherwise.  The compensated float scan also reads
-// param "blocked": lanes scan consecutive elements (BG above); 1 = one
-// transpose round (4 waves and q 8 or 16, or 8 waves and q 8), 2 = two
-// rounds of half the chunks each, in half the LDS, with registers bounded
-// for 4 waves per SIMD (4 or 8 waves, q 8 or 16).
+// Tile shape (waves x chunks per thread) of an array scan.  A tile is read,
+// scanned and written by one workgroup, so small ranges take small tiles that
+// reach every CU, and large ones large tiles (fewer look-backs).  Each line
+// lies where the two sides met; us a call:
+//   int32    4 x 8 | 8 x 16    1 M: 5.5 10.3   2 M: 6.4 7.8   4 M: 10.3 10.2
+//   float    4 x 8 | 8 x 8     2 M: 8.0 8.4    4 M: 12.6 11.9
+//            8 x 8 | tuned     4 M: 11.9 13.0  8 M: 16.7 15.3
+//   8-byte   4 x 8 | 8 x 16    1 M: 7.6 7.9    2 M: 11.3 10.7  64 M: 271 233
+// (int32 took 8 x 16 at every size, 8-byte types 4 x 4: 9.2 at 1 M, 318 at
+// 64 M.)
+//
+// Above those sizes 4-byte types take the shape of the tuning cache (key
+// "__bcmi_scan", or "__bcmi_scan_f32" for the compensated float scan; param
+// "q": 4, 8 or 16; param "waves": 4, or 8 with q = 8 or 16; param "fit_size"
+// = 0 keeps it at every size).  The compensated float scan also reads param
+// "blocked": lanes scan consecutive elements (BG above); 1 = one transpose
+// round (4 waves and q 8 or 16, or 8 waves and q 8), 2 = two rounds of half
+// the chunks each, in half the LDS, with registers bounded for 4 waves per
+// SIMD (4 or 8 waves, q 8 or 16).  Other types and generated inputs take
+// 4 x 4.
 template <typename P>
 constexpr bool comp_policy()
 {
@@ -431,6 +441,10 @@ static int run_scan_src(bcmi_queue q, const Src &src, void *out_, size_t n, cons
         // its own chunk count (fewer chunks: fewer VGPRs, more resident tiles)
         const bool comp = comp_policy<P>();
         const char *key = comp ? "__bcmi_scan_f32" : "__bcmi_scan";
+        if (tune_get(key, "fit_size", 1) != 0) {
+            if (n <= 2500000) return launch_scan<T, P, 8>(q, src, out, n, status, ini, exclusive);
+            if (comp && n <= 6000000) return launch_scan<T, P, 8, Src, 8>(q, src, out, n, status, ini, exclusive);
+        }
         const unsigned qq = tune_get(key, "q", 16);
         if constexpr (comp_policy<P>()) {
             const unsigned blocked = tune_get(key, "blocked", 0);
@@ -454,6 +468,10 @@ static int run_scan_src(bcmi_queue q, const Src &src, void *out_, size_t n, cons
         }
         if (qq == 16) return launch_scan<T, P, 16>(q, src, out, n, status, ini, exclusive);
         if (qq == 8) return launch_scan<T, P, 8>(q, src, out, n, status, ini, exclusive);
+    }
+    if constexpr (sizeof(T) == 8 && std::is_same<Src, ArraySrc<T>>::value) {
+        if (n <= 1500000) return launch_scan<T, P, 8>(q, src, out, n, status, ini, exclusive);
+        return launch_scan<T, P, 16, Src, 8>(q, src, out, n, status, ini, exclusive);
     }
     return launch_scan<T, P, 4>(q, src, out, n, status, ini, exclusive);
 }
