@@ -114,20 +114,21 @@ struct SegLds {
     Seg<typename P::CA> prefix;
 };
 
-// V consecutive keys, read or written as one access (16 or 32 bytes here;
-// 8 when 8-byte values pair with 4-byte keys)
+// V consecutive keys or values, read or written as one access (16 or 32 bytes
+// here; 8 when 8-byte values pair with 4-byte keys), aligned as the elements
+// are: keys and values may start anywhere in their allocations, at offsets of
+// their own
 template <typename KT, int V>
-struct alignas(V * sizeof(KT) >= 16 ? 16 : V * sizeof(KT)) key_chunk {
+struct key_chunk {
     KT v[V];
 };
 
 // One tile: Q 16-byte value chunks per thread, wave-striped as in the scan
 // (chunk q of lane l of wave w covers tile elements w*WSEG + q*64*V + l*V ..
-// +V-1).  FULL: the tile lies below n.  VEC: keys and values (and, for the
-// scans, the output) are 16-byte aligned, so full chunks move as vectors.
+// +V-1).  FULL: the tile lies below n, so every chunk moves as a vector.
 // The key before each chunk comes from the lane below (DPP), from lane 63
 // of the previous chunk, or, for the wave's first chunk, from memory.
-template <typename KT, typename VT, typename P, int MODE, int Q, bool VEC, bool FULL>
+template <typename KT, typename VT, typename P, int MODE, int Q, bool FULL>
 BDEV void segscan_body(SegLds<P> &L, const KT *__restrict__ keys, const VT *vals, VT *out,
                        KT *__restrict__ keys_out, size_t n, Ctrl *ctrl, uint64_t *status, VT init,
                        uint64_t *count_out, uint32_t epoch)
@@ -139,6 +140,9 @@ BDEV void segscan_body(SegLds<P> &L, const KT *__restrict__ keys, const VT *vals
     constexpr int V = 16 / sizeof(VT);
     constexpr int WSEG = Q * 64 * V;
     constexpr int TILE = 4 * WSEG;
+    // the last tile's whole chunks move as vectors too, where that costs no
+    // spills (the shapes that small ranges take)
+    constexpr bool PV = Q <= 4;
 
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const uint32_t tile = blockIdx.x;
@@ -153,7 +157,7 @@ BDEV void segscan_body(SegLds<P> &L, const KT *__restrict__ keys, const VT *vals
 #pragma unroll
     for (int q = 0; q < Q; ++q) {
         const int o = q * 64 * V + lane * V;
-        if (VEC && FULL) {
+        if (FULL || (PV && ok(q, V - 1))) {
             const key_chunk<KT, V> kq = *(const key_chunk<KT, V> *)(wk + o);
             const key_chunk<VT, V> vq = *(const key_chunk<VT, V> *)(wv + o);
 #pragma unroll
@@ -263,7 +267,7 @@ BDEV void segscan_body(SegLds<P> &L, const KT *__restrict__ keys, const VT *vals
         }
         if constexpr (MODE != SEG_RBK) {
             VT *dst = out + wstart + o;
-            if (VEC && FULL) {
+            if (FULL || (PV && ok(q, V - 1))) {
                 key_chunk<VT, V> c;
 #pragma unroll
                 for (int k = 0; k < V; ++k) c.v[k] = y[k];
@@ -307,7 +311,7 @@ BDEV T pick(const T (&a)[E], uint32_t i)
     return v[0];
 }
 
-template <typename KT, typename VT, typename P, int MODE, int Q, int NW, bool VEC, bool FULL>
+template <typename KT, typename VT, typename P, int MODE, int Q, int NW, bool FULL>
 BDEV void segscan_body_blk(SegLdsBlk<P, Q, NW> &L, const KT *__restrict__ keys, const VT *vals, VT *out,
                            KT *__restrict__ keys_out, size_t n, Ctrl *ctrl, uint64_t *status, VT init,
                            uint64_t *count_out, uint32_t epoch)
@@ -321,6 +325,7 @@ BDEV void segscan_body_blk(SegLdsBlk<P, Q, NW> &L, const KT *__restrict__ keys, 
     constexpr int E = Q * V;  // elements per lane
     constexpr int WSEG = Q * 64 * V;
     constexpr int TILE = NW * WSEG;
+    constexpr bool PV = Q <= 4;  // as above
 
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
     const uint32_t tile = blockIdx.x;
@@ -340,7 +345,7 @@ BDEV void segscan_body_blk(SegLdsBlk<P, Q, NW> &L, const KT *__restrict__ keys, 
 #pragma unroll
         for (int q = 0; q < Q; ++q) {
             const int o = q * 64 * V + lane * V;
-            if (VEC && FULL) {
+            if (FULL || (PV && sok(q, V - 1))) {
                 const key_chunk<KT, V> kq = *(const key_chunk<KT, V> *)(wk + o);
                 const key_chunk<VT, V> vq = *(const key_chunk<VT, V> *)(wv + o);
 #pragma unroll
@@ -474,7 +479,7 @@ BDEV void segscan_body_blk(SegLdsBlk<P, Q, NW> &L, const KT *__restrict__ keys, 
         for (int q = 0; q < Q; ++q) {
             const int o = q * 64 * V + lane * V;
             VT *dst = out + wstart + o;
-            if (VEC && FULL) {
+            if (FULL || (PV && sok(q, V - 1))) {
                 key_chunk<VT, V> c;
 #pragma unroll
                 for (int k = 0; k < V; ++k) c.v[k] = ys[q][k];
@@ -493,7 +498,7 @@ BDEV void segscan_body_blk(SegLdsBlk<P, Q, NW> &L, const KT *__restrict__ keys, 
 // per-tile latencies per element; 16 waves measured slower again).
 // Eight-wave workgroups are held to 128 VGPRs (4 waves per SIMD: two
 // workgroups per CU, as their LDS allows).
-template <typename KT, typename VT, typename P, int MODE, int Q, bool VEC, int NW = 4>
+template <typename KT, typename VT, typename P, int MODE, int Q, int NW = 4>
 __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 8 ? 4 : 1))) void k_segscan(const KT *__restrict__ keys, const VT *vals, VT *out,
                                                      KT *__restrict__ keys_out, size_t n, Ctrl *ctrl,
                                                      uint64_t *status, VT init, uint64_t *count_out,
@@ -505,19 +510,19 @@ __global__ __launch_bounds__(NW * 64) __attribute__((amdgpu_waves_per_eu(NW == 8
     if constexpr (sizeof(KT) == 4 && sizeof(VT) == 4 && Q <= 8) {
         __shared__ SegLdsBlk<P, Q, NW> lds;
         if (full)
-            segscan_body_blk<KT, VT, P, MODE, Q, NW, VEC, true>(lds, keys, vals, out, keys_out, n, ctrl, status,
+            segscan_body_blk<KT, VT, P, MODE, Q, NW, true>(lds, keys, vals, out, keys_out, n, ctrl, status,
                                                                 init, count_out, epoch);
         else
-            segscan_body_blk<KT, VT, P, MODE, Q, NW, VEC, false>(lds, keys, vals, out, keys_out, n, ctrl, status,
+            segscan_body_blk<KT, VT, P, MODE, Q, NW, false>(lds, keys, vals, out, keys_out, n, ctrl, status,
                                                                  init, count_out, epoch);
     } else {
         static_assert(NW == 4, "the striped form runs 4 waves");
         __shared__ SegLds<P> lds;
         if (full)
-            segscan_body<KT, VT, P, MODE, Q, VEC, true>(lds, keys, vals, out, keys_out, n, ctrl, status, init,
+            segscan_body<KT, VT, P, MODE, Q, true>(lds, keys, vals, out, keys_out, n, ctrl, status, init,
                                                         count_out, epoch);
         else
-            segscan_body<KT, VT, P, MODE, Q, VEC, false>(lds, keys, vals, out, keys_out, n, ctrl, status, init,
+            segscan_body<KT, VT, P, MODE, Q, false>(lds, keys, vals, out, keys_out, n, ctrl, status, init,
                                                          count_out, epoch);
     }
 }
@@ -528,26 +533,24 @@ static int launch_seg(bcmi_queue q, const void *keys, const void *vals, void *ou
 {
     constexpr size_t TILE = (size_t)NW * Q * 64 * (16 / sizeof(VT));
     size_t tiles = (n + TILE - 1) / TILE;
-    const bool vec = (((uintptr_t)keys | (uintptr_t)vals | (MODE == SEG_RBK ? 0 : (uintptr_t)out)) & 15) == 0;
     Epochs ep;
     BCMI_TRY(begin_lookback(q, 1, &ep));
-    if (vec)
-        BCMI_LAUNCH(q, MODE == SEG_RBK ? "reduce_by_key" : "segmented_scan",
-                    hipLaunchKernelGGL((k_segscan<KT, VT, P, MODE, Q, true, NW>), dim3((unsigned)tiles),
-                                       dim3(NW * 64), 0, q->stream, (const KT *)keys, (const VT *)vals, (VT *)out,
-                                       (KT *)keys_out, n, q->ctrl, status, ini, count_out, ep.arg(0)));
-    else
-        BCMI_LAUNCH(q, MODE == SEG_RBK ? "reduce_by_key" : "segmented_scan",
-                    hipLaunchKernelGGL((k_segscan<KT, VT, P, MODE, Q, false, NW>), dim3((unsigned)tiles),
-                                       dim3(NW * 64), 0, q->stream, (const KT *)keys, (const VT *)vals, (VT *)out,
-                                       (KT *)keys_out, n, q->ctrl, status, ini, count_out, ep.arg(0)));
+    BCMI_LAUNCH(q, MODE == SEG_RBK ? "reduce_by_key" : "segmented_scan",
+                hipLaunchKernelGGL((k_segscan<KT, VT, P, MODE, Q, NW>), dim3((unsigned)tiles), dim3(NW * 64), 0,
+                                   q->stream, (const KT *)keys, (const VT *)vals, (VT *)out, (KT *)keys_out, n,
+                                   q->ctrl, status, ini, count_out, ep.arg(0)));
     return 0;
 }
 
-// Chunks per thread from the tuning cache (key "__bcmi_reduce_by_key" or
-// "__bcmi_segscan", param "q": 2, 4 or 8) for 4-byte keys with 4-byte
-// values, and waves per workgroup (param "waves": 4, or 8 with q = 8);
-// 4 chunks and 4 waves otherwise.
+// Tile shape (waves x chunks per thread).  As in the scan, small ranges take
+// small tiles; us a call, smaller tile first:
+//   4-byte keys and values   4 x 2 | 4 x 4   10 K: 5.0 6.1 (scan 5.8 5.9)   262 K: 7.4 7.3 (6.5 6.1)
+//                            4 x 4 | 8 x 8   1 M: 10.3 10.6 (9.4 10.2)   2 M: 12.7 11.8 (13.1 11.8)
+//   8-byte values            4 x 4 | 4 x 8   262 K: 7.7 8.3   1 M: 11.4 10.7   16 M: 103 80.5 (scan 124 99.6)
+// Above those sizes 4-byte keys with 4-byte values take the shape of the
+// tuning cache (key "__bcmi_reduce_by_key" or "__bcmi_segscan", param "q": 2,
+// 4 or 8; param "waves": 4, or 8 with q = 8; param "fit_size" = 0 keeps it at
+// every size).  8-byte keys with 4-byte values take 4 x 4.
 template <typename KT, typename VT, typename P, int MODE>
 static int run_seg(bcmi_queue q, const void *keys, const void *vals, void *out, void *keys_out, size_t n,
                    const void *init, uint64_t *count_out)
@@ -561,11 +564,21 @@ static int run_seg(bcmi_queue q, const void *keys, const void *vals, void *out, 
     if (init) memcpy(&ini, init, sizeof(VT));
     if constexpr (sizeof(KT) == 4 && sizeof(VT) == 4) {
         const char *key = MODE == SEG_RBK ? "__bcmi_reduce_by_key" : "__bcmi_segscan";
+        if (tune_get(key, "fit_size", 1) != 0) {
+            if (n <= 100000)
+                return launch_seg<KT, VT, P, MODE, 2>(q, keys, vals, out, keys_out, n, status, ini, count_out);
+            if (n <= 1500000)
+                return launch_seg<KT, VT, P, MODE, 4>(q, keys, vals, out, keys_out, n, status, ini, count_out);
+        }
         const unsigned qq = tune_get(key, "q", 8);
         if (qq == 8 && tune_get(key, "waves", 4) == 8)
             return launch_seg<KT, VT, P, MODE, 8, 8>(q, keys, vals, out, keys_out, n, status, ini, count_out);
         if (qq == 8) return launch_seg<KT, VT, P, MODE, 8>(q, keys, vals, out, keys_out, n, status, ini, count_out);
         if (qq == 2) return launch_seg<KT, VT, P, MODE, 2>(q, keys, vals, out, keys_out, n, status, ini, count_out);
+    }
+    if constexpr (sizeof(VT) == 8) {
+        if (n > 500000)
+            return launch_seg<KT, VT, P, MODE, 8>(q, keys, vals, out, keys_out, n, status, ini, count_out);
     }
     return launch_seg<KT, VT, P, MODE, 4>(q, keys, vals, out, keys_out, n, status, ini, count_out);
 }
