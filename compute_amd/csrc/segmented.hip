@@ -32,16 +32,36 @@ namespace bcmi {
 
 // ------------------------------------------------------------ small path
 constexpr uint32_t kBucketMax = 64;  // largest bucket the one-pass sort finishes by insertion
+constexpr uint32_t kBinMax = 32;     // largest bin whose keys are placed by counting
+
+// The key forms of integers.
+template <typename XF>
+struct xf_is_integer : std::false_type {};
+template <typename KB>
+struct xf_is_integer<KeyXf<KB, kXfXor>> : std::true_type {};
+template <typename KB>
+struct xf_is_integer<KeyXf<KB, kXfNegXor>> : std::true_type {};
 
 // Sorts each span of segs entirely in LDS.  The keys (values) are read from
 // ksrc (vsrc) and the sorted span written to keys (vals) at the same offset;
 // the small-segment route sorts in place (ksrc == keys).
 //
-// First range-adaptive passes: with [mn, mx] the span's range of transformed
-// keys, rel(k) = (key(k) - mn) >> shift, shift chosen so rel fits 8 bits
-// (spans up to 512 keys) or 16 bits, is monotone in the key.  One or two
-// stable 8-bit LDS passes order the keys by rel; then each run of equal rel
-// (a few keys for spread-out keys: 4096 keys over 2^16 values) is finished
+// Integer keys are first dealt into bins: with [mn, mx] the span's range of
+// transformed keys, bin(k) = (key(k) - mn) >> shift, one bin per key slot
+// (up to 2048).  A returning LDS add gives each key a slot in its bin, in any
+// order; a key's place in the span is then its bin's start plus the number of
+// the bin's keys below it (by whole key, then by input position), which every
+// thread counts for its own keys, so the span goes straight to memory.
+// Spread-out keys share a bin with about one other: some 12 LDS operations a
+// pair instead of 24 for two ranked passes and the insertions (65,536 segments,
+// 69 M pairs: BEFORE -> AFTER us a run with its copies).  A bin over kBinMax
+// keys, and float keys (which crowd the bins of their largest octaves), take
+// the passes below.
+//
+// Range-adaptive passes: rel(k) = (key(k) - mn) >> shift, shift chosen so rel
+// fits 8 bits (spans up to 512 keys) or 16 bits, is monotone in the key.  One
+// or two stable 8-bit LDS passes order the keys by rel; then each run of equal
+// rel (a few keys for spread-out keys: 4096 keys over 2^16 values) is finished
 // by a stable insertion sort on the whole key, owned by the thread holding
 // the run's first slot.  If a run exceeds kBucketMax keys (clustered keys)
 // the span takes all 8-bit LSD passes in LDS instead.
@@ -55,8 +75,15 @@ __global__ __launch_bounds__(kSegSmallThreads) void k_seg_small(const KB *ksrc, 
     constexpr int TILE = kSegSmallThreads * IPT;
     __shared__ KB s_k[TILE];
     __shared__ V s_v[VB ? TILE : 1];
-    __shared__ uint32_t s_cnt[4][256];
-    __shared__ uint64_t s_peer[4][256];
+    // the passes' digit counters and peer masks, or the bins and the input
+    // positions of the binned keys
+    constexpr int NB = kSegSmallThreads * (IPT > 8 ? 8 : IPT);
+    constexpr int WORK = NB * 4 + TILE * 2 > 4 * 256 * 12 ? NB * 4 + TILE * 2 : 4 * 256 * 12;
+    __shared__ __align__(16) unsigned char s_work[WORK];
+    uint32_t(*s_cnt)[256] = (uint32_t(*)[256])s_work;
+    uint64_t(*s_peer)[256] = (uint64_t(*)[256])(s_work + 4 * 256 * 4);
+    uint32_t *s_bin = (uint32_t *)s_work;
+    uint16_t *s_idx = (uint16_t *)(s_work + NB * 4);
     __shared__ uint32_t s_wsum[4];
     __shared__ uint32_t s_uniform;
     __shared__ KB s_mn[4], s_mx[4];
@@ -82,10 +109,12 @@ __global__ __launch_bounds__(kSegSmallThreads) void k_seg_small(const KB *ksrc, 
             if (valid(j)) v[j] = vs[pos(j)];
         }
     }
-    for (int i = tid; i < 4 * 256; i += kSegSmallThreads) {
-        (&s_peer[0][0])[i] = 0;
-        (&s_cnt[0][0])[i] = 0;
-    }
+    auto clear_work = [&] {
+        for (int i = tid; i < 4 * 256 * 12 / 16; i += kSegSmallThreads)
+            ((uint4 *)s_work)[i] = make_uint4(0, 0, 0, 0);
+    };
+    static_assert(NB * 4 <= 4 * 256 * 12, "clear_work covers the bins");
+    clear_work();
 
     // one stable LDS counting pass by dig() over the register-held keys:
     // in-wave ranks, the block's digit offsets, scatter to LDS, read back in
@@ -162,10 +191,67 @@ __global__ __launch_bounds__(kSegSmallThreads) void k_seg_small(const KB *ksrc, 
             }
             return;
         }
+        const uint32_t bitlen = 64u - (uint32_t)__builtin_clzll((unsigned long long)(KB)(mx - mn));
+        // ---- bins
+        if constexpr (xf_is_integer<XF>::value) {
+            constexpr uint32_t NBITS = 31 - __builtin_clz(NB);
+            const uint32_t sh = bitlen > NBITS ? bitlen - NBITS : 0u;
+            auto bin = [&](KB x) { return (uint32_t)((KB)(xf.key(x) - mn) >> sh); };  // < NB
+            uint32_t slot[IPT];
+#pragma unroll
+            for (int j = 0; j < IPT; ++j)
+                if (valid(j)) slot[j] = atomicAdd(&s_bin[bin(k[j])], 1u);
+            block_barrier();
+            constexpr int BPT = NB / kSegSmallThreads;  // consecutive bins per thread
+            uint32_t c[BPT], tot = 0, most = 0;
+#pragma unroll
+            for (int i = 0; i < BPT; ++i) c[i] = s_bin[tid * BPT + i];
+#pragma unroll
+            for (int i = 0; i < BPT; ++i) {
+                tot += c[i];
+                most = c[i] > most ? c[i] : most;
+            }
+            uint32_t start = block_exclusive_sum256(tot, s_wsum);
+#pragma unroll
+            for (int i = 0; i < BPT; ++i) {
+                s_bin[tid * BPT + i] = start;
+                start += c[i];
+            }
+            if (!block_barrier_or(most > kBinMax)) {
+#pragma unroll
+                for (int j = 0; j < IPT; ++j) {
+                    if (!valid(j)) continue;
+                    const uint32_t dst = s_bin[bin(k[j])] + slot[j];
+                    s_k[dst] = k[j];
+                    if constexpr (VB > 0) s_v[dst] = v[j];
+                    s_idx[dst] = (uint16_t)pos(j);
+                }
+                block_barrier();
+#pragma unroll
+                for (int j = 0; j < IPT; ++j) {
+                    const uint32_t i = pos(j);
+                    if (i >= len) continue;
+                    const KB x = s_k[i];
+                    const KB tx = xf.key(x);
+                    const uint32_t b = bin(x), b0 = s_bin[b], b1 = b + 1 < (uint32_t)NB ? s_bin[b + 1] : len;
+                    uint32_t at = b0;
+                    if (b1 - b0 > 1) {
+                        const uint32_t ix = s_idx[i];
+                        for (uint32_t e = b0; e < b1; ++e) {
+                            const KB te = xf.key(s_k[e]);
+                            at += (te < tx || (te == tx && s_idx[e] < ix)) ? 1u : 0u;
+                        }
+                    }
+                    kp[at] = x;
+                    if constexpr (VB > 0) vp[at] = s_v[i];
+                }
+                return;
+            }
+            clear_work();  // the keys are still in registers, in input order
+        }
         // the leading 8 (spans up to 512 keys) or 16 bits of key - mn, as
         // one or two 8-bit passes, least significant first
         const uint32_t bits = len > 512 ? 16u : 8u;
-        const uint32_t bitlen = 64u - (uint32_t)__builtin_clzll((unsigned long long)(KB)(mx - mn));
         const uint32_t shift = bitlen > bits ? bitlen - bits : 0u;
         auto rel = [&](KB x) { return (KB)((KB)(xf.key(x) - mn) >> shift); };  // < 2^bits
         if (bits == 16) lds_pass([&](KB x) { return (uint32_t)rel(x) & 0xFFu; });
@@ -279,20 +365,24 @@ __global__ void k_seg_insertion(T *keys, typename ValT<VB>::type *vals, const Se
 enum : uint32_t { kRouteLsd = 0, kRouteMsd = 1 };
 
 // One block per histogram chunk (<= kSegChunk keys of one segment): the
-// histograms of digits [p0, p1).  With route != nullptr only chunks of
-// segments on the LSD route are counted (the others need just the top digit).
-template <typename KB, typename XF>
+// histograms of digits [p0, p0 + NP).  With route != nullptr only chunks of
+// segments on the LSD route are counted (the others need just the top digit,
+// NP = 1: 4 KB of LDS to clear and add up instead of 32 KB for 8-byte keys),
+// and none if *any_lsd says that no segment takes it.
+template <typename KB, int NP, typename XF>
 __global__ __launch_bounds__(kHistThreads) void k_seg_histogram(const KB *__restrict__ keys,
                                                                 const SegSpan *__restrict__ chunks, XF xf,
                                                                 uint32_t *__restrict__ partial, uint32_t p0,
-                                                                uint32_t p1, const uint32_t *__restrict__ route)
+                                                                const uint32_t *__restrict__ route,
+                                                                const uint32_t *__restrict__ any_lsd)
 {
     constexpr int P = sizeof(KB);
     constexpr int NW = kHistThreads / 64;
-    __shared__ uint32_t s_hist[NW][P][256];
+    __shared__ uint32_t s_hist[NW][NP][256];
+    if (route && !*any_lsd) return;
     const SegSpan c = chunks[blockIdx.x];
     if (route && route[c.idx] != kRouteLsd) return;
-    for (int i = threadIdx.x; i < NW * P * 256; i += kHistThreads) (&s_hist[0][0][0])[i] = 0;
+    for (int i = threadIdx.x; i < NW * NP * 256; i += kHistThreads) (&s_hist[0][0][0])[i] = 0;
     block_barrier();
     uint32_t(*h)[256] = s_hist[threadIdx.x >> 6];
     const KB *kc = keys + c.base;
@@ -307,14 +397,15 @@ __global__ __launch_bounds__(kHistThreads) void k_seg_histogram(const KB *__rest
 #pragma unroll
         for (int u = 0; u < U; ++u) {
             if (i0 + u * kHistThreads < c.len) {
-                const KB k = xf.key(kk[u]);
-                for (uint32_t p = p0; p < p1; ++p) atomicAdd(&h[p][(k >> (8 * p)) & 0xFF], 1u);
+                const KB k = (KB)(xf.key(kk[u]) >> (8 * p0));
+#pragma unroll
+                for (int p = 0; p < NP; ++p) atomicAdd(&h[p][(k >> (8 * p)) & 0xFF], 1u);
             }
         }
     }
     block_barrier();
-    uint32_t *dst = partial + (size_t)blockIdx.x * P * 256;
-    for (uint32_t i = p0 * 256 + threadIdx.x; i < p1 * 256; i += kHistThreads) {
+    uint32_t *dst = partial + ((size_t)blockIdx.x * P + p0) * 256;
+    for (uint32_t i = threadIdx.x; i < NP * 256; i += kHistThreads) {
         uint32_t t = 0;
 #pragma unroll
         for (int w = 0; w < NW; ++w) t += (&s_hist[w][0][0])[i];
@@ -324,14 +415,20 @@ __global__ __launch_bounds__(kHistThreads) void k_seg_histogram(const KB *__rest
 
 // grid (large segments, passes p0 + blockIdx.y): digit d of segment s summed
 // over its chunks [chunk_begin[s], chunk_begin[s+1]) and scanned into
-// exclusive offsets; with route != nullptr, LSD-route segments only.
+// exclusive offsets; with route != nullptr, LSD-route segments only.  The
+// first launch (route == nullptr) clears *any_lsd for the route kernel.
 __global__ __launch_bounds__(256) void k_seg_digit_offsets(const uint32_t *__restrict__ partial,
                                                            const uint32_t *__restrict__ chunk_begin, uint32_t passes,
                                                            uint32_t p0, uint32_t *__restrict__ seg_off,
-                                                           const uint32_t *__restrict__ route)
+                                                           const uint32_t *__restrict__ route, uint32_t *any_lsd)
 {
     __shared__ uint32_t s_wsum[4];
     const uint32_t s = blockIdx.x, p = p0 + blockIdx.y, d = threadIdx.x;
+    if (!route) {
+        if (s == 0 && d == 0) *any_lsd = 0;
+    } else if (!*any_lsd) {
+        return;
+    }
     if (route && route[s] != kRouteLsd) return;
     uint32_t c = 0;
     for (uint32_t b = chunk_begin[s]; b < chunk_begin[s + 1]; ++b) c += partial[((size_t)b * passes + p) * 256 + d];
@@ -347,10 +444,15 @@ void k_onesweep_seg(const KB *__restrict__ kin, KB *__restrict__ kout,
                                                                uint32_t pass, uint32_t passes,
                                                                const uint32_t *__restrict__ seg_off, XF xf,
                                                                Ctrl *ctrl, uint64_t *__restrict__ status,
-                                                               uint32_t back, uint32_t want)
+                                                               uint32_t back, uint32_t want,
+                                                               const uint32_t *__restrict__ any_lsd)
 {
     // the tile carries its segment's route (one load before a tile of the
     // other route exits)
+    // no segment takes this route: out after one scalar load, which the
+    // whole grid shares (a load of its own tile kept every workgroup for a
+    // memory latency, 22 us a pass over 10,807 tiles)
+    if (want == kRouteLsd && !*any_lsd) return;
     const SegTile t = tiles[blockIdx.x];
     if (t.route != want) return;  // the segment takes the other route
     const size_t b = t.base;
@@ -371,9 +473,14 @@ __global__ __launch_bounds__(kSortThreads) void k_qsweep_seg(KB *kin, KB *kout,
                                                              uint32_t pass, uint32_t passes,
                                                              const uint32_t *__restrict__ seg_off, XF xf,
                                                              Ctrl *ctrl, uint64_t *__restrict__ status,
-                                                             uint32_t back, uint32_t want)
+                                                             uint32_t back, uint32_t want,
+                                                               const uint32_t *__restrict__ any_lsd)
 {
     __shared__ QSweepLds<kSortThreads, IPT, KB, VB, 1> lds;
+    // no segment takes this route: out after one scalar load, which the
+    // whole grid shares (a load of its own tile kept every workgroup for a
+    // memory latency, 22 us a pass over 10,807 tiles)
+    if (want == kRouteLsd && !*any_lsd) return;
     const SegTile t = tiles[blockIdx.x];
     if (t.route != want) return;  // the segment takes the other route
     const uint32_t epoch = launch_epoch(ctrl, back);
@@ -403,8 +510,8 @@ __global__ __launch_bounds__(kSortThreads) void k_qsweep_seg(KB *kin, KB *kout,
 __global__ __launch_bounds__(256) void k_seg_route(const SegSpan *__restrict__ large,
                                                    const uint32_t *__restrict__ seg_off, uint32_t passes,
                                                    const uint32_t *__restrict__ slot_begin, SegSpan *groups,
-                                                   uint32_t *route, SegTile *tiles, uint32_t tile_len, uint32_t cap,
-                                                   uint32_t enable)
+                                                   uint32_t *route, uint32_t *any_lsd, SegTile *tiles,
+                                                   uint32_t tile_len, uint32_t cap, uint32_t enable)
 {
     __shared__ uint32_t s_start[257];
     __shared__ uint32_t s_jump[2][257];
@@ -455,7 +562,10 @@ __global__ __launch_bounds__(256) void k_seg_route(const SegSpan *__restrict__ l
     }
     const bool msd = enable && !big && ngroups <= b1 - b0;
     const uint32_t rt = msd ? kRouteMsd : kRouteLsd;
-    if (d == 0) route[s] = rt;
+    if (d == 0) {
+        route[s] = rt;
+        if (!msd) *any_lsd = 1;  // the same value from every such segment
+    }
     if (msd && m) groups[b0 + before + mbcnt(bal)] = SegSpan{sg.base + sd, s_start[nx] - sd, 0};
     for (uint32_t i = (msd ? b0 + ngroups : b0) + d; i < b1; i += 256) groups[i] = SegSpan{0, 0, 0};
     const uint32_t nt = (uint32_t)(((uint64_t)sg.len + tile_len - 1) / tile_len);
@@ -501,6 +611,7 @@ struct bcmi_segplan_s {
     bcmi::SegSpan *large = nullptr;
     bcmi::SegSpan *chunks = nullptr;
     uint32_t *route = nullptr;       // per large segment: kRouteLsd / kRouteMsd (set on the device)
+    uint32_t *any_lsd = nullptr;     // whether any segment's route is kRouteLsd (set on the device)
     uint32_t *slot_begin = nullptr;  // per large segment: first group slot (nlarge + 1 entries)
     bcmi::SegSpan *groups = nullptr; // MSD route groups (written on the device)
     uint32_t *chunk_begin = nullptr;
@@ -578,27 +689,27 @@ static int run_plan_large(bcmi_queue q, bcmi_segplan pl, KB *keys, typename ValT
         // (MSD needs two digits or more); the other digits are counted only
         // for segments on the LSD route
         BCMI_LAUNCH(q, "segsort_histogram",
-                    hipLaunchKernelGGL((k_seg_histogram<KB, XF>), dim3(pl->nchunks), dim3(kHistThreads), 0, q->stream,
-                                       keys, pl->chunks, xf, pl->partial, (uint32_t)(P - 1), (uint32_t)P,
-                                       (const uint32_t *)nullptr));
+                    hipLaunchKernelGGL((k_seg_histogram<KB, 1, XF>), dim3(pl->nchunks), dim3(kHistThreads), 0,
+                                       q->stream, keys, pl->chunks, xf, pl->partial, (uint32_t)(P - 1),
+                                       (const uint32_t *)nullptr, (const uint32_t *)pl->any_lsd));
         BCMI_LAUNCH(q, "segsort_digit_offsets",
                     hipLaunchKernelGGL(k_seg_digit_offsets, dim3(pl->nlarge, 1), dim3(256), 0, q->stream, pl->partial,
                                        pl->chunk_begin, (uint32_t)P, (uint32_t)(P - 1), pl->seg_off,
-                                       (const uint32_t *)nullptr));
+                                       (const uint32_t *)nullptr, pl->any_lsd));
         BCMI_LAUNCH(q, "segsort_route",
                     hipLaunchKernelGGL(k_seg_route, dim3(pl->nlarge), dim3(256), 0, q->stream, pl->large, pl->seg_off,
-                                       (uint32_t)P, pl->slot_begin, pl->groups, pl->route, pl->tiles,
+                                       (uint32_t)P, pl->slot_begin, pl->groups, pl->route, pl->any_lsd, pl->tiles,
                                        (uint32_t)(kSortThreads * IPTL), (uint32_t)(kSegSmallThreads << pl->small_cls),
                                        (uint32_t)(P >= 2 && pl->msd)));
-        if (P >= 2) {
+        if constexpr (P >= 2) {
             BCMI_LAUNCH(q, "segsort_histogram",
-                        hipLaunchKernelGGL((k_seg_histogram<KB, XF>), dim3(pl->nchunks), dim3(kHistThreads), 0,
-                                           q->stream, keys, pl->chunks, xf, pl->partial, 0u, (uint32_t)(P - 1),
-                                           (const uint32_t *)pl->route));
+                        hipLaunchKernelGGL((k_seg_histogram<KB, P - 1, XF>), dim3(pl->nchunks), dim3(kHistThreads), 0,
+                                           q->stream, keys, pl->chunks, xf, pl->partial, 0u,
+                                           (const uint32_t *)pl->route, (const uint32_t *)pl->any_lsd));
             BCMI_LAUNCH(q, "segsort_digit_offsets",
                         hipLaunchKernelGGL(k_seg_digit_offsets, dim3(pl->nlarge, P - 1), dim3(256), 0, q->stream,
                                            pl->partial, pl->chunk_begin, (uint32_t)P, 0u, pl->seg_off,
-                                           (const uint32_t *)pl->route));
+                                           (const uint32_t *)pl->route, pl->any_lsd));
         }
         uint64_t *status;
         BCMI_TRY(status_array(q, (size_t)pl->ntiles * 256, &status));
@@ -613,13 +724,13 @@ static int run_plan_large(bcmi_queue q, bcmi_segplan pl, KB *keys, typename ValT
                             hipLaunchKernelGGL((k_qsweep_seg<KB, VB, IPTL, XF>), dim3(pl->ntiles),              \
                                                dim3(kSortThreads), 0, q->stream, KS, KD, VS, VD, pl->tiles,     \
                                                SHIFT, PASS, (uint32_t)P, pl->seg_off, xf, q->ctrl, status,      \
-                                               BACK, WANT));                                                    \
+                                               BACK, WANT, (const uint32_t *)pl->any_lsd));                                                    \
             else                                                                                                \
                 BCMI_LAUNCH(q, NAME,                                                                            \
                             hipLaunchKernelGGL((k_onesweep_seg<KB, VB, IPTL, XF>), dim3(pl->ntiles),            \
                                                dim3(kSortThreads), 0, q->stream, KS, KD, VS, VD, pl->tiles,     \
                                                SHIFT, PASS, (uint32_t)P, pl->seg_off, xf, q->ctrl, status,      \
-                                               BACK, WANT));                                                    \
+                                               BACK, WANT, (const uint32_t *)pl->any_lsd));                                                    \
         } while (0)
         BCMI_SEG_PASS("segsort_onesweep_msd", keys, (KB *)pl->ktmp, vals, (V *)pl->vtmp, (uint32_t)(8 * (P - 1)),
                       (uint32_t)(P - 1), ep.arg(0), (uint32_t)kRouteMsd);
@@ -782,7 +893,7 @@ extern "C" int bcmi_segmented_plan_create(bcmi_queue q, int key_dtype, size_t va
     o_tiles = off; off += al256(tiles.size() * sizeof(SegTile));
     o_partial = off; off += al256(chunks.size() * (size_t)kb * 256 * 4);
     o_segoff = off; off += al256(large.size() * (size_t)kb * 256 * 4);
-    const size_t o_route = off; off += al256(large.size() * sizeof(uint32_t));
+    const size_t o_route = off; off += al256((large.size() + 1) * sizeof(uint32_t));
     const size_t o_sb = off; off += al256(slot_begin.size() * sizeof(uint32_t));
     const size_t o_groups = off; off += al256((size_t)slot_begin.back() * sizeof(SegSpan));
     // temporaries cover the elements of large segments at their own offsets
@@ -804,6 +915,7 @@ extern "C" int bcmi_segmented_plan_create(bcmi_queue q, int key_dtype, size_t va
     pl->partial = (uint32_t *)(m + o_partial);
     pl->seg_off = (uint32_t *)(m + o_segoff);
     pl->route = (uint32_t *)(m + o_route);
+    pl->any_lsd = pl->route + large.size();
     pl->slot_begin = (uint32_t *)(m + o_sb);
     pl->groups = (SegSpan *)(m + o_groups);
     pl->nslots = slot_begin.back();
