@@ -1,0 +1,8 @@
+// Instantiation unit of segmented.hpp.
+#include "segmented.hpp"
+
+namespace bcmi {
+
+BCMI_SEGPLAN_SIGNATURE(segplan_run_u64) { return run_plan_vb<uint64_t>(q, pl, keys, vals); }
+
+}  // namespace bcmi
