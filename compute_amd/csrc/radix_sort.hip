@@ -23,32 +23,41 @@
 
 namespace bcmi {
 
-// One block of 1024 threads per pass: thread (slice, d) sums digit d over a
-// quarter of the partial histograms, the slices are combined in LDS and the
-// 256 totals scanned into exclusive digit offsets.  A pass whose digit is the
-// same in all n keys is marked in ctrl->single.
+// kOffsetBlocks blocks of 1024 threads per pass: wave w of block (p, part)
+// sums 64 digits over every 16th partial histogram, the waves are combined in
+// LDS and the digits scanned; the digits of earlier parts come from their
+// blocks' totals, passed on as tagged words (a part waits for earlier blocks
+// only).  A pass whose digit is the same in all n keys is marked in
+// ctrl->single: its block passes on ~0, which no total reaches.  One block per
+// pass read up to 1 MB of partials through one CU's cache: 15 us for 33.5 M
+// keys with values, 8.5 us for 2^27 keys.
 __global__ __launch_bounds__(1024) void k_digit_offsets(const uint32_t *__restrict__ partial, uint32_t nparts,
-                                                        uint32_t passes, uint32_t n, Ctrl *ctrl)
+                                                        uint32_t passes, uint32_t n, Ctrl *ctrl, uint64_t *status,
+                                                        uint32_t ep)
 {
-    __shared__ uint32_t s_part[4][256];
-    __shared__ uint32_t s_wsum[4];
-    const uint32_t p = blockIdx.x, d = threadIdx.x & 255, slice = threadIdx.x >> 8;
+    __shared__ uint32_t s_part[16][64];
+    const uint32_t p = blockIdx.x / kOffsetBlocks, part = blockIdx.x % kOffsetBlocks;
+    const uint32_t lane = threadIdx.x & 63, w = threadIdx.x >> 6, d = part * 64 + lane;
     uint32_t c = 0;
 #pragma unroll 8
-    for (uint32_t b = slice; b < nparts; b += 4) c += partial[((size_t)b * passes + p) * 256 + d];
-    s_part[slice][d] = c;
+    for (uint32_t b = w; b < nparts; b += 16) c += partial[((size_t)b * passes + p) * 256 + d];
+    s_part[w][lane] = c;
     block_barrier();
-    const uint32_t lane = d & 63, w = d >> 6;
-    c = s_part[0][d] + s_part[1][d] + s_part[2][d] + s_part[3][d];
-    uint32_t inc = wave_inclusive_scan(c, 0u, [](uint32_t a, uint32_t b) { return a + b; });
-    if (slice == 0 && lane == 63) s_wsum[w] = inc;
-    const int single = block_barrier_or(c == n);
-    if (threadIdx.x == 0) ctrl->single[p] = single ? 1u : 0u;
-    if (slice == 0) {
-        uint32_t pre = 0;
-        for (uint32_t i = 0; i < w; ++i) pre += s_wsum[i];
-        ctrl->offsets[p][d] = pre + inc - c;
-    }
+    if (w != 0) return;
+#pragma unroll
+    for (int i = 1; i < 16; ++i) c += s_part[i][lane];
+    const uint32_t epoch = launch_epoch(ctrl, ep);
+    const uint32_t inc = wave_inclusive_scan(c, 0u, [](uint32_t a, uint32_t b) { return a + b; });
+    bool single = ballot(c == n) != 0;
+    if (lane == 0) lb_publish(status, blockIdx.x, epoch, LB_A, single ? ~0u : readlane(inc, 63));
+    uint32_t before = 0, spins = 0;
+    if (lane < part)
+        while (lb_read(status, blockIdx.x - part + lane, epoch, before) == LB_X)
+            if (spin_expired(ctrl, spins)) break;
+    single = single || ballot(before == ~0u) != 0;
+    before = wave_reduce(before == ~0u ? n : before, 0u, [](uint32_t a, uint32_t b) { return a + b; });
+    ctrl->offsets[p][d] = before + inc - c;
+    if (part == kOffsetBlocks - 1 && lane == 0) ctrl->single[p] = single ? 1u : 0u;
 }
 
 // ------------------------------------------------------- insertion sort

@@ -169,7 +169,9 @@ static int launch_histogram(bcmi_queue q, const HistShape &hs, uint32_t hblocks,
 
 // Sums the histogram blocks' partials per digit, scans them into
 // ctrl->offsets and marks the passes that move nothing (radix_sort.hip).
-__global__ void k_digit_offsets(const uint32_t *partial, uint32_t nparts, uint32_t passes, uint32_t n, Ctrl *ctrl);
+constexpr uint32_t kOffsetBlocks = 4;
+__global__ void k_digit_offsets(const uint32_t *partial, uint32_t nparts, uint32_t passes, uint32_t n, Ctrl *ctrl,
+                                uint64_t *status, uint32_t ep);
 __global__ void k_clear_words(uint64_t *p, size_t n);
 
 inline size_t align256(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -238,16 +240,16 @@ static int radix_sort_xf(bcmi_queue q, void *keys_, void *vals_, uint32_t n, XF 
     V *vtmp = (V *)(scr + pbytes + kbytes);
 
     BCMI_TRY(launch_histogram(q, hs, hblocks, keys, n, head, xf, partial));
-    BCMI_LAUNCH(q, "radix_digit_offsets",
-                hipLaunchKernelGGL(k_digit_offsets, dim3(P), dim3(1024), 0, q->stream, partial, hblocks,
-                                   (uint32_t)P, n, q->ctrl));
     Epochs ep;
-    BCMI_TRY(begin_lookback(q, P, &ep));
+    BCMI_TRY(begin_lookback(q, P + 1, &ep));
+    BCMI_LAUNCH(q, "radix_digit_offsets",
+                hipLaunchKernelGGL(k_digit_offsets, dim3(P * kOffsetBlocks), dim3(1024), 0, q->stream, partial, hblocks,
+                                   (uint32_t)P, n, q->ctrl, status, ep.arg(0)));
     for (int p = 0; p < P; ++p)
         BCMI_LAUNCH(q, "radix_onesweep",
                     hipLaunchKernelGGL((k_qsweep<TH, IPT, KB, VB, SPLIT, LB, WPE, XF, CBG>), dim3(tiles), dim3(TH), 0,
                                        q->stream, keys, ktmp, vals, vtmp, n, (uint32_t)p, xf, q->ctrl, status,
-                                       ep.arg((uint32_t)p), (uint32_t)xrun));
+                                       ep.arg((uint32_t)p + 1), (uint32_t)xrun));
     if (P & 1) {
         // one pass (8-bit keys): the result is in the temporary
         BCMI_HIP(hipMemcpyAsync(keys, ktmp, (size_t)n * sizeof(KB), hipMemcpyDeviceToDevice, q->stream));
