@@ -31,6 +31,8 @@ what varies is the tile shape and the work per thread):
                                        also the MSD group size), MSD route for large segments on or off, keys
                                        per thread of a large segment's tile (8-byte elements: 12 or 24),
                                        quarter-wave ranking in the large passes
+The sorts, scans and reduce_by_key take smaller tiles for smaller ranges, by
+size; param "fit_size" = 0 of their keys keeps the tuned shape at every size.
 
     python -m compute_amd.autotune [--out PATH] [--log2n-sort 27] ...
 """
