@@ -148,6 +148,22 @@ int begin_lookback(bcmi_queue q, int launches, Epochs *epochs)
     return 0;
 }
 
+int side_stream(bcmi_queue q, int i, SideStream **side)
+{
+    SideStream &s = q->side[i];
+    *side = nullptr;
+    if (!s.join) {
+        hipStreamCaptureStatus cap = hipStreamCaptureStatusNone;
+        BCMI_HIP(hipStreamIsCapturing(q->stream, &cap));
+        if (cap != hipStreamCaptureStatusNone) return 0;
+        if (!s.stream) BCMI_HIP(hipStreamCreateWithFlags(&s.stream, hipStreamNonBlocking));
+        if (!s.fork) BCMI_HIP(hipEventCreateWithFlags(&s.fork, hipEventDisableTiming));
+        BCMI_HIP(hipEventCreateWithFlags(&s.join, hipEventDisableTiming));
+    }
+    *side = &s;
+    return 0;
+}
+
 static hipEvent_t pool_event(bcmi_queue q)
 {
     if (!q->event_pool.empty()) {
@@ -308,6 +324,11 @@ int bcmi_queue_destroy(bcmi_queue q)
     if (q->status) (void)hipFree(q->status);
     if (q->ctrl) (void)hipFree(q->ctrl);
     if (q->pinned) (void)hipHostFree(q->pinned);
+    for (SideStream &s : q->side) {
+        if (s.fork) (void)hipEventDestroy(s.fork);
+        if (s.join) (void)hipEventDestroy(s.join);
+        if (s.stream) (void)hipStreamDestroy(s.stream);
+    }
     if (q->stream) (void)hipStreamDestroy(q->stream);
     delete q;
     return 0;

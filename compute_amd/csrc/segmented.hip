@@ -115,22 +115,18 @@ extern "C" int bcmi_segmented_plan_create(bcmi_queue q, int key_dtype, size_t va
             return s2;
         }
     }
-    // the plan's streams (default priority) and their events, where there is
-    // something to run beside the large segments' top-digit route
-    bool any_small = pl->ninsert != 0;
-    for (int c = 0; c < 5; ++c) any_small = any_small || pl->nsmall[c] != 0;
-    auto branch = [](hipStream_t *st, hipEvent_t *fork, hipEvent_t *join) {
-        hipError_t r = hipStreamCreateWithFlags(st, hipStreamNonBlocking);
-        if (r == hipSuccess) r = hipEventCreateWithFlags(fork, hipEventDisableTiming);
-        if (r == hipSuccess) r = hipEventCreateWithFlags(join, hipEventDisableTiming);
-        return r;
-    };
-    hipError_t e2 = hipSuccess;
-    if (any_small && pl->nlarge) e2 = branch(&pl->aux, &pl->fork, &pl->join);
-    if (e2 == hipSuccess && pl->ntiles >= kForkLsdTiles) e2 = branch(&pl->lsd, &pl->lsd_fork, &pl->lsd_join);
-    if (e2 != hipSuccess) {
+    // the queue's side streams, where there is something to run beside the
+    // large segments' top-digit route
+    for (int c = 0; c < 5; ++c) pl->fork_small = pl->fork_small || pl->nsmall[c] != 0;
+    pl->fork_small = (pl->fork_small || pl->ninsert != 0) && pl->nlarge;
+    // 1-byte keys have no top-digit route
+    pl->fork_lsd = kb >= 2 && pl->ntiles >= (pl->fork_small ? kForkLsdTilesMixed : kForkLsdTiles);
+    SideStream *side;
+    int s3 = pl->fork_small ? side_stream(q, kSideSmall, &side) : 0;
+    if (!s3 && pl->fork_lsd) s3 = side_stream(q, kSideLsd, &side);
+    if (s3) {
         bcmi_segmented_plan_destroy(pl);
-        return hip_fail(e2, "segmented plan stream", __FILE__, __LINE__);
+        return s3;
     }
     *plan = pl;
     return 0;
@@ -140,10 +136,6 @@ extern "C" int bcmi_segmented_plan_destroy(bcmi_segplan plan)
 {
     if (!plan) return 0;
     (void)hipSetDevice(plan->device);
-    for (hipEvent_t ev : {plan->fork, plan->join, plan->lsd_fork, plan->lsd_join})
-        if (ev) (void)hipEventDestroy(ev);
-    for (hipStream_t st : {plan->aux, plan->lsd})
-        if (st) (void)hipStreamDestroy(st);
     if (plan->mem) BCMI_HIP(hipFree(plan->mem));
     delete plan;
     return 0;

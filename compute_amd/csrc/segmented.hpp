@@ -622,16 +622,17 @@ struct bcmi_segplan_s {
     uint32_t *seg_off = nullptr;
     void *ktmp = nullptr;
     void *vtmp = nullptr;
-    // the small segments, and (in plans of kForkLsdTiles tiles) the large
-    // ones' all-digits route, are sorted on streams of the plan's own,
-    // concurrently with the top-digit route (the three touch disjoint
-    // elements, tiles and status words): forked from and joined back into the
-    // queue's stream, so a graph capture records the branches
-    hipStream_t aux = nullptr, lsd = nullptr;
-    hipEvent_t fork = nullptr, join = nullptr, lsd_fork = nullptr, lsd_join = nullptr;
+    // whether the small segments, and the large ones' all-digits passes, are
+    // sorted on the queue's side streams, concurrently with the top-digit
+    // route (the three touch disjoint elements, tiles and status words):
+    // forked from and joined back into the queue's stream, so a graph capture
+    // records the branches
+    bool fork_small = false, fork_lsd = false;
 };
 
 namespace bcmi {
+
+enum : int { kSideSmall = 0, kSideLsd = 1 };  // bcmi_queue_s::side
 
 // Keys per thread of the large segments' onesweep tiles (256 threads): 8,
 // 12 or 16 by element width; for 8-byte keys or values the tuning cache
@@ -681,26 +682,37 @@ static int run_plan_small(bcmi_queue q, bcmi_segplan pl, KB *keys, typename ValT
     return 0;
 }
 
-// Tiles from which the all-digits route goes to a stream of its own.
-// Usually no segment takes it, and then each of its launches is a grid that
-// leaves at once, but at the pace at which a CU can place workgroups of 51 KB
-// of LDS: 22 us a pass over 10,807 tiles, 8 passes for 8-byte keys; and
-// where segments do take it, it is half of the work.  65,536 segments with the
-// copies: float keys 2407 -> 2253 us, uint64 keys 0.929 -> 0.922 of the time
-// before both changes.  Smaller plans are bound by the launches themselves,
-// which the event calls would only add to.
-constexpr uint32_t kForkLsdTiles = 1024;
+// Tiles from which the all-digits passes go to a side stream, beside the
+// top-digit route.  Where a plan's segments take both routes the two overlap;
+// where none takes this one, its launches do (grids that leave at once, at the
+// pace at which a CU can place workgroups of 51 KB of LDS: 22 us a pass over
+// 10,437 tiles).  Fork and join cost about 20 us, which a plan whose segments
+// are alike gets nothing for, so its line lies where they are a percent or
+// two; a plan with small segments too has lengths of all kinds, which take
+// both routes, and forks from half as many tiles on.  us a run with the copies,
+// one stream | two:
+//   10 segments of 2^22,    10,240 tiles of uint32 keys below 100: 1449 1470
+//   6 segments of 2^22,       4096 tiles of uint64 keys: 1841 1860
+//   500 segments of 20,000,   2500 tiles of uint32 keys below 100: 327 349
+//   65,536 of all lengths,  10,437 tiles of uint64 keys: 1267 1256, 13,718 of float: 2316 2121
+//   30,000 of all lengths,    4800 tiles of uint64 keys:  604  589,   6300 of float: 1100 1034
+//   16,000 of all lengths,    2480 tiles of uint64 keys:  342  333,   3225 of float:  714  701
+//   10,000 of 300 and 300 of 30,000, 1500 tiles of uint64 keys: 237 231, 2400 of uint32: 163 171
+// The other digits' histograms stay on the queue's stream: beside the
+// top-digit groups their few blocks land on the CUs that those leave free,
+// several on one (206 -> 405 us for 500 segments of 20,000 uint64 keys).
+constexpr uint32_t kForkLsdTiles = 6400, kForkLsdTilesMixed = 3200;
 
 // The large segments: top-digit route decision, MSD groups, LSD passes (on
-// stream ls: q->stream, or the plan's own with the decision waited for).
+// q->stream, or on the side stream lsd with the decision waited for).
 template <typename KB, int VB, typename XF, int IPTL>
 static int run_plan_large(bcmi_queue q, bcmi_segplan pl, KB *keys, typename ValT<VB>::type *vals, XF xf,
-                          bool *lsd_forked)
+                          SideStream *lsd, bool *lsd_forked)
 {
     using V = typename ValT<VB>::type;
     constexpr int P = sizeof(KB);
     if (pl->nlarge) {
-        const hipStream_t ls = pl->lsd && !q->profile ? pl->lsd : q->stream;
+        const hipStream_t ls = lsd ? lsd->stream : q->stream;
         // the top digit's histogram and offsets decide each segment's route
         // (MSD needs two digits or more); the other digits are counted only
         // for segments on the LSD route
@@ -723,20 +735,20 @@ static int run_plan_large(bcmi_queue q, bcmi_segplan pl, KB *keys, typename ValT
         BCMI_TRY(status_array(q, (size_t)pl->ntiles * 256, &status));
         Epochs ep;
         BCMI_TRY(begin_lookback(q, P + 1, &ep));
-        if (ls != q->stream) {
-            BCMI_HIP(hipEventRecord(pl->lsd_fork, q->stream));
-            BCMI_HIP(hipStreamWaitEvent(ls, pl->lsd_fork, 0));
-            *lsd_forked = true;
-        }
         if constexpr (P >= 2) {
             BCMI_LAUNCH(q, "segsort_histogram",
                         hipLaunchKernelGGL((k_seg_histogram<KB, P - 1, XF>), dim3(pl->nchunks), dim3(kHistThreads), 0,
-                                           ls, keys, pl->chunks, xf, pl->partial, 0u,
+                                           q->stream, keys, pl->chunks, xf, pl->partial, 0u,
                                            (const uint32_t *)pl->route, (const uint32_t *)pl->any_lsd));
             BCMI_LAUNCH(q, "segsort_digit_offsets",
-                        hipLaunchKernelGGL(k_seg_digit_offsets, dim3(pl->nlarge, P - 1), dim3(256), 0, ls, pl->partial,
-                                           pl->chunk_begin, (uint32_t)P, 0u, pl->seg_off,
+                        hipLaunchKernelGGL(k_seg_digit_offsets, dim3(pl->nlarge, P - 1), dim3(256), 0, q->stream,
+                                           pl->partial, pl->chunk_begin, (uint32_t)P, 0u, pl->seg_off,
                                            (const uint32_t *)pl->route, pl->any_lsd));
+        }
+        if (lsd) {
+            BCMI_HIP(hipEventRecord(lsd->fork, q->stream));
+            BCMI_HIP(hipStreamWaitEvent(ls, lsd->fork, 0));
+            *lsd_forked = true;
         }
         // MSD route: top-digit partition into the temporaries ...
         // (param "qrank" = 1: the quarter-wave pass body)
@@ -796,15 +808,17 @@ static int run_plan_xf(bcmi_queue q, bcmi_segplan pl, void *keys_, void *vals_, 
     using V = typename ValT<VB>::type;
     KB *keys = (KB *)keys_;
     V *vals = (V *)vals_;
-    // the small segments go to the plan's stream when there is large work
-    // to overlap them with (not while the queue profiles kernels: its
-    // per-kernel times are taken on the queue's stream)
-    const bool forked = pl->aux != nullptr && !q->profile;
-    if (forked) {
-        BCMI_HIP(hipEventRecord(pl->fork, q->stream));
-        BCMI_HIP(hipStreamWaitEvent(pl->aux, pl->fork, 0));
+    // the small segments go to a side stream when there is large work to
+    // overlap them with (not while the queue profiles kernels: its per-kernel
+    // times are taken on the queue's stream)
+    SideStream *small = nullptr, *lsd = nullptr;
+    if (pl->fork_small && !q->profile) BCMI_TRY(side_stream(q, kSideSmall, &small));
+    if (pl->fork_lsd && !q->profile) BCMI_TRY(side_stream(q, kSideLsd, &lsd));
+    if (small) {
+        BCMI_HIP(hipEventRecord(small->fork, q->stream));
+        BCMI_HIP(hipStreamWaitEvent(small->stream, small->fork, 0));
     }
-    int st = run_plan_small<KB, VB, XF>(q, pl, keys, vals, xf, forked ? pl->aux : q->stream);
+    int st = run_plan_small<KB, VB, XF>(q, pl, keys, vals, xf, small ? small->stream : q->stream);
     bool lsd_forked = false;
     if (!st) {
         constexpr int SB = (int)sizeof(KB) > VB ? (int)sizeof(KB) : VB;
@@ -813,21 +827,21 @@ static int run_plan_xf(bcmi_queue q, bcmi_segplan pl, void *keys_, void *vals_, 
         bool ran = false;
         if constexpr (SB == 8) {
             if (pl->ipt_large == 24) {
-                st = run_plan_large<KB, VB, XF, 24>(q, pl, keys, vals, xf, &lsd_forked);
+                st = run_plan_large<KB, VB, XF, 24>(q, pl, keys, vals, xf, lsd, &lsd_forked);
                 ran = true;
             }
         }
-        if (!ran) st = run_plan_large<KB, VB, XF, IPTL>(q, pl, keys, vals, xf, &lsd_forked);
+        if (!ran) st = run_plan_large<KB, VB, XF, IPTL>(q, pl, keys, vals, xf, lsd, &lsd_forked);
     }
     // the joins are recorded whatever happened, so that a capture is never
     // left with a branch outside the queue's stream
-    auto join = [&](hipEvent_t ev, hipStream_t from) {
-        hipError_t e = hipEventRecord(ev, from);
-        if (e == hipSuccess) e = hipStreamWaitEvent(q->stream, ev, 0);
+    auto join = [&](SideStream *side) {
+        hipError_t e = hipEventRecord(side->join, side->stream);
+        if (e == hipSuccess) e = hipStreamWaitEvent(q->stream, side->join, 0);
         if (e != hipSuccess && !st) st = hip_fail(e, "segmented sort: join", __FILE__, __LINE__);
     };
-    if (forked) join(pl->join, pl->aux);
-    if (lsd_forked) join(pl->lsd_join, pl->lsd);
+    if (small) join(small);
+    if (lsd_forked) join(lsd);
     return st;
 }
 
