@@ -549,8 +549,10 @@ static int launch_select(bcmi_queue q, const T *in, void *out_a, void *out_b, si
     // few hundred: one tile per CU leaves its loads, ranks and stores in
     // series.  us a call, quarter tiles first: copy_if of int32 1 M: 6.5 11.3,
     // 4 M: 12.0 14.9, 8 M: 19.6 19.0; of int64 1 M: 8.2 9.2, 2 M: 11.2 11.1;
-    // partition_copy of int32 4 M: 14.4 17.0, 8 M: 22.9 22.4.
-    if (n <= (size_t)SelShape<T>::TILE * (sizeof(T) == 8 ? 192 : 384))
+    // of int16 3 M: 9.4 9.7, 4 M: 11.8 10.8; of uint8 3 M: 9.1 9.2, 4 M: 11.4
+    // 10.3 (unique of uint8 3 M: 8.5 8.9, 6 M: 12.4 10.1); partition_copy of
+    // int32 4 M: 14.4 17.0, 8 M: 22.9 22.4.
+    if (n <= (size_t)SelShape<T>::TILE * (sizeof(T) == 4 ? 384 : 192))
         return launch_select_div<T, MODE, 4>(q, in, out_a, out_b, n, p, count_out);
     return launch_select_div<T, MODE, 1>(q, in, out_a, out_b, n, p, count_out);
 }

@@ -71,7 +71,7 @@ def test_by_key_lines(queue, vdt, n, koff, voff):
 
 
 @pytest.mark.parametrize("dt,line", [("int32", 384 * 16384), ("float32", 384 * 16384), ("int64", 192 * 8192),
-                                     ("uint8", 384 * 16384)])
+                                     ("uint8", 384 * 16384), ("uint8", 192 * 16384), ("int16", 192 * 16384)])
 @pytest.mark.parametrize("off", [0, 1])
 def test_select_lines(queue, dt, line, off):
     rng = np.random.default_rng(off)
