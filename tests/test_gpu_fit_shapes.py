@@ -148,3 +148,20 @@ def test_tuned_shapes_at_small_sizes(queue, key, shapes):
     finally:
         for p, v in saved.items():
             ca.check(L.bcmi_tune_set(key.encode(), p.encode(), v))
+
+
+@pytest.mark.parametrize("dt", ["int8", "uint8", "int16", "uint16"])
+def test_narrow_reduce_off_the_grid(queue, dt):
+    """Every offset to a 16-byte boundary, ranges that end before it included."""
+    rng = np.random.default_rng(2)
+    x = rng.integers(np.iinfo(dt).min, np.iinfo(dt).max, 70000, dtype=dt, endpoint=True)
+    d = ca.DeviceArray.from_host(x, queue)
+    out = ca.DeviceArray(2, dt, queue)
+    code = ca.DTYPE[x.dtype]
+    for off in range(17):
+        for n in (1, 2, 7, 14, 15, 16, 17, 31, 33, 8191, 65537):
+            s = x[off:off + n]
+            ca.check(ca.lib().bcmi_reduce(queue.h, code, ca.PLUS, d.at(off), n, None, out.ptr, None, ca.COMPENSATED))
+            ca.check(ca.lib().bcmi_reduce(queue.h, code, ca.MIN, d.at(off), n, None, out.at(1), None, ca.COMPENSATED))
+            got = out.to_host(queue)
+            assert got[0] == s.sum(dtype=dt) and got[1] == s.min(), (off, n)
