@@ -108,3 +108,32 @@ def test_plans_share_a_queues_side_streams():
             assert np.array_equal(d.to_host(q), e), rep
     for q in (built, other):
         q.close()
+
+
+@pytest.mark.parametrize("dt", ["uint8", "int16", "uint32", "int32", "uint64", "int64"])
+def test_crowded_bins(queue, dt):
+    """Small integer segments on both sides of what the bins hold (32 keys
+    each): as many values as the segment just needs, one more and one fewer,
+    away from zero and at the type's ends; one bin of 31 to 34 keys among
+    spread ones; keys spread over octaves; equal keys in input order."""
+    rng = np.random.default_rng(np.dtype(dt).itemsize)
+    info, parts = np.iinfo(dt), []
+    for n in (33, 63, 64, 65, 96, 97, 255, 256, 257, 511, 512, 513, 1023, 1024, 1025, 2047, 2048):
+        for values in sorted({max(1, -(-n // 32) + d) for d in (-1, 0, 1)} | {2}):
+            lo = (info.min, 7, info.max - values + 1)[rng.integers(3)]
+            k = (np.arange(n) % values).astype(dt) + np.array(lo, dt)  # as even as it gets
+            parts += [k, rng.permutation(k)]
+        for crowd in (31, 32, 33, 34):
+            k = rng.integers(info.min, info.max, n, dtype=dt, endpoint=True)
+            k[rng.permutation(n)[:crowd]] = 3
+            parts.append(k)
+        parts.append(np.exp2(rng.uniform(0, np.log2(float(info.max)) - 0.01, n)).astype(dt))
+    off = np.concatenate([[0], np.cumsum([p.size for p in parts])]).astype(np.uint64)
+    k = np.concatenate(parts)
+    v = np.arange(k.size, dtype=np.uint32)
+    for desc in (False, True):
+        dk, dv = ca.DeviceArray.from_host(k, queue), ca.DeviceArray.from_host(v, queue)
+        ca.segmented_sort(queue, dk, dv, off, descending=desc)
+        ek, ev = O.segmented_sort(k, v, off, descending=desc)
+        assert np.array_equal(dk.to_host(queue), ek), desc
+        assert np.array_equal(dv.to_host(queue), ev), desc
