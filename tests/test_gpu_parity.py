@@ -750,12 +750,13 @@ def test_scan_tunable_shapes(queue, waves, q):
     its bound with both accumulator forms, whole and partial tiles."""
     L = ca.lib()
     keys_t = ("__bcmi_scan", "__bcmi_scan_f32")
-    params = ("waves", "q", "acc", "blocked")
+    params = ("waves", "q", "acc", "blocked", "fit_size")
     saved = {k: [_tune_get(k, p) for p in params] for k in keys_t}
     try:
         for k in keys_t:
             ca.check(L.bcmi_tune_set(k.encode(), b"waves", waves))
             ca.check(L.bcmi_tune_set(k.encode(), b"q", q))
+            ca.check(L.bcmi_tune_set(k.encode(), b"fit_size", 0))  # this shape at every size
         ca.check(L.bcmi_tune_set(b"__bcmi_scan_f32", b"blocked", 0))  # the striped layout
         for n in (1, 5000, 65536 * 3 + 7, (1 << 21) + 13):
             x = RNG.integers(-1000, 1000, n).astype(np.int32)
@@ -783,7 +784,7 @@ def test_scan_tunable_shapes(queue, waves, q):
                 assert np.all(np.abs(fo.to_host(queue).astype(np.float64) - dd) <= _scan_err_bound(xf, dd)), (n, acc)
     finally:
         for k, vals_ in saved.items():
-            for p, val, d in zip(params, vals_, (4, 16, 1, 0)):
+            for p, val, d in zip(params, vals_, (4, 16, 1, 0, 1)):
                 ca.check(L.bcmi_tune_set(k.encode(), p.encode(), val if val != 0xFFFFFFFF else d))
 
 
@@ -797,11 +798,12 @@ def test_scan_blocked_layout(queue, waves, q, blocked):
     double-double oracle."""
     L = ca.lib()
     key = "__bcmi_scan_f32"
-    params = ("waves", "q", "acc", "blocked")
+    params = ("waves", "q", "acc", "blocked", "fit_size")
     saved = [_tune_get(key, p) for p in params]
     try:
         ca.check(L.bcmi_tune_set(key.encode(), b"waves", waves))
         ca.check(L.bcmi_tune_set(key.encode(), b"q", q))
+        ca.check(L.bcmi_tune_set(key.encode(), b"fit_size", 0))  # this shape at every size
         ca.check(L.bcmi_tune_set(key.encode(), b"blocked", blocked))
         for n in (1, 77, 5000, 65536 * 3 + 7, (1 << 21) + 13):
             x = O.gen_lognormal_f32(n)
@@ -831,7 +833,7 @@ def test_scan_blocked_layout(queue, waves, q, blocked):
                     got = fo.to_host(queue)[2:].astype(np.float64)
                     assert np.all(np.abs(got - dd) <= _scan_err_bound(x[1:1 + m], dd)), (n, acc, "unaligned")
     finally:
-        for p, val, d in zip(params, saved, (4, 16, 1, 0)):
+        for p, val, d in zip(params, saved, (4, 16, 1, 0, 1)):
             ca.check(L.bcmi_tune_set(key.encode(), p.encode(), val if val != 0xFFFFFFFF else d))
 
 
@@ -842,12 +844,13 @@ def test_segmented_scan_tunable_shapes(queue, waves, q):
     sums within the compensated bound, whole and partial tiles."""
     L = ca.lib()
     keys_t = ("__bcmi_reduce_by_key", "__bcmi_segscan")
-    params = ("waves", "q")
+    params = ("waves", "q", "fit_size")
     saved = {k: [_tune_get(k, p) for p in params] for k in keys_t}
     try:
         for k in keys_t:
             ca.check(L.bcmi_tune_set(k.encode(), b"waves", waves))
             ca.check(L.bcmi_tune_set(k.encode(), b"q", q))
+            ca.check(L.bcmi_tune_set(k.encode(), b"fit_size", 0))  # this shape at every size
         for n in (1, 4097, 100003, (1 << 20) + 17):
             lens = RNG.integers(1, 70, n)
             keys = np.repeat(np.arange(lens.size, dtype=np.int32), lens)[:n]
@@ -876,21 +879,25 @@ def test_segmented_scan_tunable_shapes(queue, waves, q):
             assert np.all(np.abs(fo.to_host(queue).astype(np.float64) - dd) <= bound), n
     finally:
         for k, vals_ in saved.items():
-            for p, val, d in zip(params, vals_, (4, 8)):
+            for p, val, d in zip(params, vals_, (4, 8, 1)):
                 ca.check(L.bcmi_tune_set(k.encode(), p.encode(), val if val != 0xFFFFFFFF else d))
 
 
+@pytest.mark.parametrize("fit", [0, 1])
 @pytest.mark.parametrize("acc", [0, 1])
-def test_float_accumulator_policies(queue, acc):
+def test_float_accumulator_policies(queue, acc, fit):
     """Both float accumulator policies the tuner may pick (1: FP64
     accumulators, 0: TwoSum FP32 pairs) meet the compensated bound for the
-    scan, reduce_by_key and the segmented scan, on whole and partial tiles."""
+    scan, reduce_by_key and the segmented scan, on whole and partial tiles, in
+    the shapes for their sizes and in the tuned ones."""
     L = ca.lib()
     keys_t = ("__bcmi_scan_f32", "__bcmi_reduce_by_key", "__bcmi_segscan")
-    saved = [_tune_get(k, "acc") for k in keys_t]
+    params = ("acc", "fit_size")
+    saved = [[_tune_get(k, p) for p in params] for k in keys_t]
     try:
         for k in keys_t:
             ca.check(L.bcmi_tune_set(k.encode(), b"acc", acc))
+            ca.check(L.bcmi_tune_set(k.encode(), b"fit_size", fit))
         for n in (4096 * 3 + 5, (1 << 20) + 17):
             x = O.gen_lognormal_f32(n)
             out = ca.DeviceArray(n, np.float32, queue)
@@ -912,8 +919,9 @@ def test_float_accumulator_policies(queue, acc):
                     2.0 ** -50 * np.cumsum(np.abs(vals.astype(np.float64)))
                 assert np.all(np.abs(out.to_host(queue).astype(np.float64) - dd) <= bound), (n, excl)
     finally:
-        for k, val in zip(keys_t, saved):
-            ca.check(L.bcmi_tune_set(k.encode(), b"acc", val if val != 0xFFFFFFFF else 1))
+        for k, vals_ in zip(keys_t, saved):
+            for p, val in zip(params, vals_):
+                ca.check(L.bcmi_tune_set(k.encode(), p.encode(), val if val != 0xFFFFFFFF else 1))
 
 
 @pytest.mark.parametrize("small_max,msd,ipt,qrank", [(2, 1, 12, 0), (3, 0, 12, 0), (0, 1, 12, 0), (3, 1, 24, 0),
