@@ -43,3 +43,62 @@ def test_sort_shape_lines(queue, dt, vb, off):
         assert got[0 if off else n].tobytes() == k[0 if off else n].tobytes()  # the element beside the range
         if vb:
             assert np.array_equal(dv.to_host(queue), ev), n
+
+
+# sizes of every tile shape, the largest ones the tuned, XCD-grouped shapes'
+IDLE = [("uint32", 0, [16385, 300007, 3000017, 13000027]), ("uint32", 4, [8193, 1200007, 5200003]),
+        ("uint64", 0, [8193, 600011, 6100007]), ("uint64", 4, [8193, 1200007, 6100007]),
+        ("int32", 8, [8193, 1200007, 6100007]), ("uint32", 1, [30011]), ("int32", 2, [30011]), ("uint32", 16, [30011]),
+        ("uint64", 16, [30011]), ("uint16", 0, [16385, 1000003]), ("int16", 4, [30011]), ("uint8", 4, [30011])]
+# byte positions that vary: none; first one at an odd position (the later
+# passes read the other array); an odd number of them (one idle pass copies)
+MOVING = {1: [(), (0,)], 2: [(), (0,), (1,)], 4: [(), (1, 2), (0, 1, 3), (1,), (3,), (0, 2)],
+          8: [(), (1, 2), (0, 3, 5), (1,), (2, 4, 6, 7), (1, 2, 3, 4, 5, 6)]}
+
+
+def _moving_keys(dt, n, moving, rng):
+    w = np.dtype(dt).itemsize
+    k = np.full(n, 0x81A5C37E5B9D4F01 & ((1 << 8 * w) - 1), "u%d" % w)
+    b = k.view(np.uint8).reshape(n, w)
+    for i in moving:
+        b[:, i] = rng.integers(0, 256, n, dtype=np.uint8)
+    return k.view(dt)
+
+
+@pytest.mark.parametrize("dt,vb,sizes", IDLE)
+def test_sort_with_idle_passes(queue, dt, vb, sizes):
+    """Keys with bytes that are the same in all of them: the passes over those
+    bytes are left out, in every tile shape and value width."""
+    rng = np.random.default_rng(vb)
+    for n in sizes:
+        for i, moving in enumerate(MOVING[np.dtype(dt).itemsize]):
+            if n > 2000000 and i not in (1, 2):
+                continue
+            k = _moving_keys(dt, n, moving, rng)
+            order = np.arange(n, dtype=np.uint32)
+            v = rng.integers(0, 256, (n, vb), dtype=np.uint8)
+            for desc in (False, True) if n < 100000 else (bool(i & 1),):
+                d = ca.DeviceArray.from_host(k, queue)
+                dv = ca.DeviceArray.from_host(v.reshape(-1), queue) if vb else None
+                ca.check(ca.lib().bcmi_sort(queue.h, ca.RADIX_SORT, ca.DTYPE[k.dtype], d.ptr, dv.ptr if vb else None,
+                                            vb, n, int(desc)))
+                ek, eo = O.radix_order_sort(k, order, descending=desc)
+                assert np.array_equal(d.to_host(queue), ek), (n, moving, desc)
+                if vb:
+                    assert np.array_equal(dv.to_host(queue).reshape(n, vb), v[eo]), (n, moving, desc)
+
+
+@pytest.mark.parametrize("dt,vb", [("uint32", 0), ("uint64", 4)])
+def test_noalloc_sort_with_idle_passes(queue, dt, vb):
+    rng = np.random.default_rng(vb + 1)
+    for n in (1000003, 20011):
+        for moving in MOVING[np.dtype(dt).itemsize]:
+            k = _moving_keys(dt, n, moving, rng)
+            v = np.arange(n, dtype=np.uint32)
+            d, dv = ca.DeviceArray.from_host(k, queue), ca.DeviceArray.from_host(v, queue)
+            ca.check(ca.lib().bcmi_sort_noalloc(queue.h, ca.RADIX_SORT, ca.DTYPE[k.dtype], d.ptr,
+                                                dv.ptr if vb else None, vb, n, 0))
+            ek, ev = O.radix_order_sort(k, v)
+            assert np.array_equal(d.to_host(queue), ek), (n, moving)
+            if vb:
+                assert np.array_equal(dv.to_host(queue), ev), (n, moving)
