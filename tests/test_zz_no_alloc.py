@@ -32,7 +32,8 @@ def _both(q, api, dtype, keys, vals, vb, desc):
     return out
 
 
-@pytest.mark.parametrize("n1,n2", [(3_000_017, 70_001), (1 << 20, 4097)])
+# (up to 16384 keys, 8192 of 8 bytes or with values, the sort takes no scratch)
+@pytest.mark.parametrize("n1,n2", [(3_000_017, 70_001), (1 << 20, 16_411), (1 << 20, 4097)])
 def test_noalloc_sort_keys_matches_sort(queue, n1, n2):
     for n in (n1, n2):  # second call smaller
         k = O.gen_sort_u32(n, seed=0xB0057001 + n)
@@ -54,7 +55,7 @@ def test_noalloc_sort_by_key_float_matches_sort(queue):
 
 def test_noalloc_sort_u64_keys_u32_values_matches_sort(queue):
     rng = np.random.default_rng(7)
-    for n in (1_000_003, 5000):
+    for n in (1_000_003, 8_209, 5000):
         k = rng.integers(0, 2 ** 63, n, dtype=np.uint64)
         k[rng.integers(0, n, n // 10)] = k[0]
         v = np.arange(n, dtype=np.uint32)
