@@ -157,8 +157,9 @@ BDEV void part_publish(uint64_t *status, uint32_t block, uint32_t epoch, Pt p)
     lb_publish(status, block, epoch, LB_A, b);
 }
 
-// A bounded wait (every block but the last publishes without waiting, and
-// blocks are dispatched in order, so it ends).
+// A bounded wait, as a look-back's: every block but the last publishes without
+// waiting, and the last is dispatched after the others of its XCD and runs
+// beside those of the rest, so it ends.
 template <typename Pt>
 BDEV Pt part_wait(const uint64_t *status, uint32_t block, uint32_t epoch, Ctrl *ctrl)
 {

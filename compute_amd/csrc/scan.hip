@@ -226,7 +226,9 @@ BDEV void scan_body(ScanLds<P, NW> &L, uint32_t *blk, const Src src, T *out, siz
     auto okb = [&](int e) { return FULL || (int64_t)(lane * Q * V + e) < rem; };
     constexpr bool BLK = BG > 0;
     // the last tile's whole chunks move as vectors too, where that costs no
-    // spills (the shapes that small ranges take)
+    // spills (1- and 2-byte elements and generated inputs; the shapes of 4- and
+    // 8-byte arrays have 8 chunks or more, and their last tile, which is the
+    // only one of a short range, moves element by element)
     constexpr bool PV = Q <= 4;
     uint32_t *wblk = blk + w * RowShape<Q, BLK ? BG : Q>::WORDS;
 

@@ -55,12 +55,20 @@ struct xf_is_integer<KeyXf<KB, kXfNegXor>> : std::true_type {};
 // order; a key's place in the span is then its bin's start plus the number of
 // the bin's keys below it (by whole key, then by input position), which every
 // thread counts for its own keys, so the span goes straight to memory.
-// Spread-out keys share a bin with about one other: some 12 LDS operations a
-// pair instead of 24 for two ranked passes and the insertions (with the flag
-// below and the top digit's own histogram, 65,536 segments of 69 M uint64 +
-// uint32 pairs and their copies: 1449 -> 1346 us).  A bin over kBinMax
-// keys, and float keys (which crowd the bins of their largest octaves), take
-// the passes below.
+// Spread-out keys share a bin with about one other: 24 LDS instructions a pair
+// and 90 LDS cycles a wave's pairs, instead of 37 and 194 for two ranked passes
+// and the insertions (SQ_INSTS_LDS, SQ_LDS_IDX_ACTIVE; spans of 2000 uint64 +
+// uint32 pairs).  A bin over kBinMax keys, and float keys (which crowd the bins
+// of their largest octaves), take the passes below; a span that tried has lost
+// the adds, which take turns on the crowded bin, and the scan.  us a run with
+// the copies, passes alone | bins first:
+//   spread keys   100,000 x 30 uint32 + uint32: 149 105   20,000 x 512: 124 63
+//                 6000 x 2048 uint64 + uint32: 123 112
+//   crowded keys  20,000 x 512 uint32 + uint32 of e^U(0, 22): 236 267, of two
+//                 values: 298 323; 6000 x 2048 uint64 in 30 clusters: 743 768
+// Foreseeing the failure did not pay: the range's size against the length cost
+// spread keys of short spans 3-4 %, a ballot over a sample of the keys 5-15 %,
+// giving up on the first full slot 2 % (the adds' returns are waited for).
 //
 // Range-adaptive passes: rel(k) = (key(k) - mn) >> shift, shift chosen so rel
 // fits 8 bits (spans up to 512 keys) or 16 bits, is monotone in the key.  One
@@ -451,13 +459,13 @@ void k_onesweep_seg(const KB *__restrict__ kin, KB *__restrict__ kout,
                                                                uint32_t back, uint32_t want,
                                                                const uint32_t *__restrict__ any_lsd)
 {
-    // the tile carries its segment's route (one load before a tile of the
-    // other route exits)
     // no segment takes this route: out after one scalar load, which the
     // whole grid shares
     if (want == kRouteLsd && !*any_lsd) return;
+    // the tile carries its segment's route (one load before a tile of the
+    // other route exits)
     const SegTile t = tiles[blockIdx.x];
-    if (t.route != want) return;  // the segment takes the other route
+    if (t.route != want) return;
     const size_t b = t.base;
     onesweep_tile<KB, VB, IPT, kRankLdsMask, XF>(kin + b, kout + b, VB ? vin + b : vin, VB ? vout + b : vout, t.len,
                                              t.tile, shift, seg_off + ((size_t)t.seg * passes + pass) * 256, xf,
@@ -480,11 +488,9 @@ __global__ __launch_bounds__(kSortThreads) void k_qsweep_seg(KB *kin, KB *kout,
                                                                const uint32_t *__restrict__ any_lsd)
 {
     __shared__ QSweepLds<kSortThreads, IPT, KB, VB, 1> lds;
-    // no segment takes this route: out after one scalar load, which the
-    // whole grid shares
-    if (want == kRouteLsd && !*any_lsd) return;
+    if (want == kRouteLsd && !*any_lsd) return;  // as above
     const SegTile t = tiles[blockIdx.x];
-    if (t.route != want) return;  // the segment takes the other route
+    if (t.route != want) return;
     const uint32_t epoch = launch_epoch(ctrl, back);
     const size_t b = t.base;
     const uint32_t *goff = seg_off + ((size_t)t.seg * passes + pass) * 256;

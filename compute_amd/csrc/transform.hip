@@ -50,9 +50,10 @@ struct BinOp {
 // last whole chunk in the thread that would have had the next one: one launch
 // for any n.  vec16 is aligned as its elements are: a wave's chunks are one
 // contiguous 1 KB either way, and off the 16-byte grid it only touches one
-// line more.  Bound by HBM from a few MB on; saxpy us a call: 4 M floats 9.1 ->
-// 7.3, 10 M 26.5 -> 19 (a second launch served the tail), 1001 floats off the
-// grid 9.6 -> 4.1 (the element-wise path that served such operands).
+// line more.  Bound by HBM from a few MB on.  us a call, before -> now: saxpy of
+// 4,000,003 floats 7.9 -> 6.6, 10,000,019 from memory 26.5 -> 24.8 (a second
+// launch served the tail), 1001 one element off the grid 11.0 -> 4.3 (a third
+// the head); 200 M int32 at unlike offsets 499 -> 429 (element by element).
 template <typename T, typename F, int U>
 __global__ __launch_bounds__(kTfThreads) void k_transform(const T *__restrict__ a, const T *__restrict__ b,
                                                           T *__restrict__ out, size_t n, F f)
